@@ -64,6 +64,26 @@ def test_dequant_bit_exact(backend, orc, dtype, rows, k):
     torch.cuda.synchronize()
 
 
+@pytest.mark.parametrize("dtype,rows,k,row0,n", [
+    (Q8_0, 16400, 64, 7, 16390), (Q6_K, 2100, 1280, 3, 2090), (IQ3, 530, 2304, 100, 301),
+    (Q5_K, 40, 1281, 15, 17), (Q4_K, 33, 1026, 0, 33), (Q4_K, 3000, 1024, 1999, 1)])
+def test_dequant_windows_bit_exact(backend, orc, dtype, rows, k, row0, n):
+    """Row windows that start and end inside a 16-row group, from whole items
+    per block down to one row per block, ragged rows, and an output that is
+    only 4-byte aligned."""
+    import torch
+    say(f"dequant window dtype={dtype} rows={rows} k={k} [{row0}, +{n})")
+    w = syn.make_blocks(dtype, rows, k, seed=rows + k)
+    h = backend.upload_weight(dtype, w, k, rows)
+    ref = orc.dequant_rows(dtype, w[row0:row0 + n], k).view(np.uint32)
+    for off in (0, 1):
+        buf = torch.full((n * k + 8,), 7.0, device="cuda")
+        h.dequant_rows(row0, n, buf[off:off + n * k])
+        got = buf.cpu().numpy()
+        assert np.array_equal(got[off:off + n * k].reshape(n, k).view(np.uint32), ref)
+        assert (got[:off] == 7.0).all() and (got[off + n * k:] == 7.0).all()
+
+
 @pytest.mark.parametrize("dtype,E,f,k", [(IQ3, 5, 32, 512), (Q4_K, 3, 48, 256), (IQ3, 3, 24, 256)])
 def test_dequant_experts_bit_exact(backend, orc, dtype, E, f, k):
     # stacked experts: rows per expert a multiple of 16 (quad layout, experts
