@@ -21,33 +21,21 @@
 //
 // Tiling (bf16): a block computes 160 weight rows x 256 tokens (18944 rows
 // x 512 tokens -> 238 blocks, one round on 256 CUs).  K advances 64
-// elements (one Q4_K group) per stage.  Batches longer than 128 tokens take
-// the direct-X kernel (X fragments straight from L2 into the multiply
-// waves' registers), shorter ones the ring kernel (X through LDS).
+// elements (one Q4_K group) per stage, X fragments come straight from L2 into
+// the multiply waves' registers.  Batches of up to 128 tokens take
+// gq_gemm_quad.hip's kernel instead.
 // int8 (k_gemm_i8_direct): 160 rows x 256 tokens, W nibbles straight to
 // int8 MFMA, per-32 scaling on the VALU.
+#include <algorithm>
 #include <type_traits>
 
-#include "gq_device.h"
+#include "gq_gemm_dev.h"
 #include "gq_internal.h"
 #include "../../include/gq.h"
 
 namespace gq {
 
-typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
-typedef float f32x4_t __attribute__((ext_vector_type(4)));
-typedef int i32x4_t __attribute__((ext_vector_type(4)));
-
 constexpr int BM = 160, BN = 256, BK = 64;
-constexpr int WM = 80, WN = 128;  // per-wave tile
-constexpr int TM = WM / 16, TN = WN / 16;
-
-// fp32 -> bf16 bits, round to nearest even (NaN kept quiet).
-__device__ __forceinline__ uint32_t f2bf(float f) {
-  const uint32_t u = __float_as_uint(f);
-  if ((u & 0x7fffffffu) > 0x7f800000u) return (u >> 16) | 0x40u;
-  return (u + 0x7fffu + ((u >> 16) & 1u)) >> 16;
-}
 
 // ----------------------------------------------------------- prepasses
 // X fp32 [n][k] -> bf16 in MFMA B-operand fragments: fragment (token tile
@@ -86,59 +74,12 @@ __global__ void k_x_to_bf16_frag(const float *X, int n, int npad, int k, int kpa
   *(uint4 *)(out + 8 * i) = make_uint4(o[0], o[1], o[2], o[3]);
 }
 
-// ----------------------------------------------------------- bf16 kernel
-// Producer / consumer: 512 threads.  Waves 0-3 only multiply: each owns an
-// 80-row x 128-token tile (5 x 8 MFMA tiles) of the 160 x 256 block tile.
-// Waves 4-7 only move and dequantize data, straight from memory to LDS
-// (global_load_lds_dwordx4, no registers):
-//   * waves 4-5 fetch the raw Q4_K units of the block's 160 rows (ggml
-//     order, 144 B per row per 256 k), one unit (4 stages of 64 k) ahead;
-//   * all four fetch the X tile (256 tokens x 64 bf16) one stage ahead and
-//     dequantize the next stage's W tile (d*sc*q - dmin*m, bf16).
-// LDS tiles are fragment-major: MFMA operand (ks, t) -- 16 rows or tokens x
-// 32 k -- is 64 lane slots of 16 B (lane l: row / token 16t + l%16, k
-// 32ks + 8(l/16) .. +8), so every operand read is a conflict-free 128-bit
-// load of consecutive slots and every X load writes a whole fragment.
-// Rings (2 slots each): dequantized W, X, raw W units (152 KiB).  One
-// barrier per stage.  A wave's waits count only its own loads (in issue
-// order), so the long-lived unit loads are issued after each stage's X
-// loads and only waves 4-5 carry them.
-constexpr int FR16 = 512;                     // bf16 per 1 KiB fragment
-
-typedef __attribute__((address_space(3))) void lds_void_t;
-
-// s_waitcnt vmcnt(N), leaving the other counters alone (gfx9 encoding).
-template <int N>
-__device__ __forceinline__ void wait_vm() {
-  __builtin_amdgcn_s_waitcnt((N & 15) | ((N >> 4) << 14) | (0x7 << 4) | (0xF << 8));
-}
-__device__ __forceinline__ void wait_lgkm0() { __builtin_amdgcn_s_waitcnt(0xC07F); }
-
-__device__ __forceinline__ void dma16(const void *g, void *lds) {
-  __builtin_amdgcn_global_load_lds(g, (lds_void_t *)lds, 16, 0, 0);
-}
-
 // LDS reads written as asm and waited for inside: the compiler, seeing
 // loads straight to LDS still outstanding, would otherwise wait for all of
 // them (vmcnt(0)) before any LDS read; the callers wait for exactly the
 // loads they read.
 typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
-__device__ __forceinline__ void lds_read2(const uint4 *p0, const uint4 *p1, uint4 &a, uint4 &b) {
-  const uint32_t a0 = (uint32_t)(uintptr_t)(lds_void_t *)p0;
-  const uint32_t a1 = (uint32_t)(uintptr_t)(lds_void_t *)p1;
-  u32x4_t x, y;
-  asm volatile(
-      "ds_read_b128 %0, %2\n\t"
-      "ds_read_b128 %1, %3\n\t"
-      "s_waitcnt lgkmcnt(0)"
-      : "=&v"(x), "=&v"(y)
-      : "v"(a0), "v"(a1)
-      : "memory");
-  a = make_uint4(x[0], x[1], x[2], x[3]);
-  b = make_uint4(y[0], y[1], y[2], y[3]);
-}
-
-// Two / four 16-byte LDS reads, one wait.
+// Two 16-byte LDS reads, one wait.
 __device__ __forceinline__ void lds_read2_a(const uint32_t (&ad)[2], uint4 (&v)[2]) {
   u32x4_t x0, x1;
   asm volatile(
@@ -151,23 +92,6 @@ __device__ __forceinline__ void lds_read2_a(const uint32_t (&ad)[2], uint4 (&v)[
   v[0] = make_uint4(x0[0], x0[1], x0[2], x0[3]);
   v[1] = make_uint4(x1[0], x1[1], x1[2], x1[3]);
 }
-__device__ __forceinline__ void lds_read4(const uint32_t (&ad)[4], uint4 (&v)[4]) {
-  u32x4_t x0, x1, x2, x3;
-  asm volatile(
-      "ds_read_b128 %0, %4\n\t"
-      "ds_read_b128 %1, %5\n\t"
-      "ds_read_b128 %2, %6\n\t"
-      "ds_read_b128 %3, %7\n\t"
-      "s_waitcnt lgkmcnt(0)"
-      : "=&v"(x0), "=&v"(x1), "=&v"(x2), "=&v"(x3)
-      : "v"(ad[0]), "v"(ad[1]), "v"(ad[2]), "v"(ad[3])
-      : "memory");
-  v[0] = make_uint4(x0[0], x0[1], x0[2], x0[3]);
-  v[1] = make_uint4(x1[0], x1[1], x1[2], x1[3]);
-  v[2] = make_uint4(x2[0], x2[1], x2[2], x2[3]);
-  v[3] = make_uint4(x3[0], x3[1], x3[2], x3[3]);
-}
-
 // Six 16-byte LDS reads, one wait.
 __device__ __forceinline__ void lds_read6(const uint32_t (&ad)[6], uint4 (&v)[6]) {
   u32x4_t x0, x1, x2, x3, x4, x5;
@@ -190,19 +114,6 @@ __device__ __forceinline__ void lds_read6(const uint32_t (&ad)[6], uint4 (&v)[6]
   v[5] = make_uint4(x5[0], x5[1], x5[2], x5[3]);
 }
 
-// Byte K of w (0..255) as float: one v_cvt_f32_ubyteK.  Written as asm
-// because the compiler otherwise folds a preceding nibble mask into a
-// v_bfe per element.
-template <int K>
-__device__ __forceinline__ float cvt_ubyte(uint32_t w) {
-  float f;
-  if constexpr (K == 0) asm("v_cvt_f32_ubyte0 %0, %1" : "=v"(f) : "v"(w));
-  else if constexpr (K == 1) asm("v_cvt_f32_ubyte1 %0, %1" : "=v"(f) : "v"(w));
-  else if constexpr (K == 2) asm("v_cvt_f32_ubyte2 %0, %1" : "=v"(f) : "v"(w));
-  else asm("v_cvt_f32_ubyte3 %0, %1" : "=v"(f) : "v"(w));
-  return f;
-}
-
 // get_scale_min_k4 (src/quant/q4_k.rs:26-35) without branches: both forms,
 // then a select on j < 4.
 __device__ __forceinline__ void scale_min_k4_sel(int j, uint32_t s0, uint32_t s1, uint32_t s2,
@@ -213,13 +124,6 @@ __device__ __forceinline__ void scale_min_k4_sel(int j, uint32_t s0, uint32_t s1
   const uint32_t hi_sc = (b & 0xFu) | ((c >> 6) << 4), hi_m = (b >> 4) | ((a >> 6) << 4);
   sc = j < 4 ? lo_sc : hi_sc;
   m = j < 4 ? lo_m : hi_m;
-}
-
-typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
-
-__device__ __forceinline__ uint32_t pack_bf16(float a, float b) {
-  const bf16x2_t v = {(__bf16)a, (__bf16)b};  // v_cvt_pk_bf16_f32: round to nearest even
-  return __builtin_bit_cast(uint32_t, v);
 }
 
 // ----------------------------------------------------------- bf16 GEMM weights
@@ -351,291 +255,6 @@ __global__ void k_gemm_records(Layout L, const uint8_t *body, const uint16_t *dd
   }
 }
 
-// ----------------------------------------------------------- bf16 kernel, ring pipeline
-// Block tile TBM rows x TBN tokens, 512 threads.  Waves 0-3 multiply: each
-// owns an 80 x 128 tile (5 x 8 MFMA tiles) and reads fragment-major LDS
-// operands (MFMA operand (ks, t), 16 rows or tokens x 32 k, is 64 lane slots
-// of 16 B: conflict-free 128-bit reads).  Waves 4-7 produce:
-//   * each fetches, two stages ahead, the stage records of its own TBM / 4
-//     rows into a ring private to the wave and dequantizes them (Q4_K:
-//     d*sc*q - dmin*m; Q6_K: d*sc*(q - 32); both rounded to bf16, RNE) into
-//     the next A tile, so it waits only for its own loads;
-//   * together they fetch the X fragments (bf16, written by a pre-pass in
-//     fragment order) into an NXR-slot ring, NXR - 1 stages ahead.
-// Loads go straight to LDS (global_load_lds_dwordx4); a producer's LDS
-// reads are inline asm with their own waits (a plain LDS read would make
-// the compiler first drain every outstanding load to LDS, the ones just
-// issued included).  One barrier per stage.
-// Blocks: (row tile, token tile, K split).  A launch covers up to
-// GEMM_MAX_SEG matrices sharing the input (row tiles numbered across them);
-// with ksplit > 1 a block covers stages [S*s/ksplit, S*(s+1)/ksplit) and
-// writes a partial product, which gemm_reduce sums in a fixed order.
-
-// Workgroups are dealt to the 8 XCDs round-robin by id (id % 8).  The
-// GEMM's block index is renumbered so that each XCD takes a contiguous range
-// of it: the token tiles (and K splits) of one row tile then run on one XCD
-// and read its W tile through the same L2.
-__device__ __forceinline__ int xcd_block(int id, int n) {
-  const int x = id & 7, j = id >> 3, q = n >> 3, r = n & 7;
-  return x * q + min(x, r) + j;
-}
-
-template <int TBM, int TBN, int NXR, int FMT>
-struct Ring {
-  static constexpr int AT_ = TBM / 16, BT_ = TBN / 16;
-  static constexpr int A_FR_ = 2 * AT_, B_FR_ = 2 * BT_;
-  static constexpr int C = GemmFmt<FMT>::C;    // 16-byte chunks per stage record
-  static constexpr int PROWS = TBM / 4;        // rows per producer wave
-  static constexpr int WSLOTS = C * PROWS;     // W chunks per producer wave per stage
-  static constexpr int WINS = (WSLOTS + 63) / 64;
-  static constexpr int XPW = B_FR_ / 4;        // X fragment loads per producer wave per stage
-  static constexpr int WGM = TBM / WM;         // multiply waves along the rows
-  static_assert(WGM * (TBN / WN) == 4, "4 multiply waves");
-  static constexpr int TASKS = 4 * PROWS;      // 16-element dequant tasks per producer wave
-  static constexpr int ROUNDS = (TASKS + 63) / 64;
-  static_assert(ROUNDS == 2 || ROUNDS == 3, "2 or 3 dequant rounds");
-  // W ring slots: 2 suffice (stage kt + 2 is fetched into the slot stage kt
-  // was dequantized from, one iteration earlier); a third where LDS allows
-  // keeps a fetch off the slot read in the iteration just before.
-  static constexpr size_t LDS2 = (size_t)2 * A_FR_ * FR16 * 2 + (size_t)NXR * B_FR_ * FR16 * 2 +
-                                 (size_t)4 * 2 * WSLOTS * 16;
-  static constexpr int WR = LDS2 + (size_t)4 * WSLOTS * 16 <= 163840 ? 3 : 2;
-};
-
-template <int TBM, int TBN, int NXR, int FMT>
-__global__ __launch_bounds__(512) void k_gemm_bf16_ring(GemmArgs a) {
-  using R = Ring<TBM, TBN, NXR, FMT>;
-  constexpr int AT_ = R::AT_, BT_ = R::BT_, PROWS = R::PROWS, WSLOTS = R::WSLOTS, C = R::C;
-  constexpr int WINS = R::WINS, XPW = R::XPW, WR = R::WR;
-  __shared__ __align__(16) uint16_t As[2][R::A_FR_ * FR16];
-  __shared__ __align__(16) uint16_t Xs[NXR][R::B_FR_ * FR16];
-  __shared__ __align__(16) uint8_t Wg[4][WR][WSLOTS * 16];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int b = xcd_block(blockIdx.x, gridDim.x), split = b % a.ksplit, rest = b / a.ksplit;
-  const int ntile = rest % a.ntiles, tile = rest / a.ntiles;
-  GemmSeg sg = a.seg[0];
-#pragma unroll
-  for (int i = 1; i < GEMM_MAX_SEG; i++)
-    if (i < a.nseg && tile >= a.seg[i].tile_begin) sg = a.seg[i];
-  const int m0 = (tile - sg.tile_begin) * TBM, n0 = ntile * TBN, rows = sg.rows;
-  const int stages_all = a.kpad / BK;
-  const int s0 = (int)((long)stages_all * split / a.ksplit);
-  const int stages = (int)((long)stages_all * (split + 1) / a.ksplit) - s0, last = stages - 1;
-  const long row_stride = (long)(stages_all / 4) * gemm_unit_bytes(FMT);
-  const bool mma = wave < 4;
-
-  if (!mma) {
-    const int pw = wave - 4;
-    const int ksteps = a.kpad / 32;
-    const uint16_t *xsrc = a.xb + ((long)(n0 / 16) * ksteps * 64 + lane) * 8;
-    // W chunk slots of this wave: q = 64 i + lane (q < WSLOTS): row
-    // PROWS * pw + q / C, chunk q % C of the stage record.
-    const uint8_t *wsrc[WINS];
-    int wc[WINS];
-#pragma unroll
-    for (int i = 0; i < WINS; i++) {
-      const int q = min(64 * i + lane, WSLOTS - 1);
-      const int row = min(m0 + PROWS * pw + q / C, rows - 1);
-      wsrc[i] = sg.rec + (long)row * row_stride;
-      wc[i] = q % C;
-    }
-    auto issue_x = [&](int s) {  // X fragments of local stage s (clamped) into slot s % NXR
-      const int sc = s0 + min(s, last);
-#pragma unroll
-      for (int qd = 0; qd < XPW; qd++) {
-        const int f = XPW * pw + qd, nt = f % BT_, ks = f / BT_;
-        dma16(xsrc + ((long)nt * ksteps + 2 * sc + ks) * 512, &Xs[s % NXR][f * FR16]);
-      }
-    };
-    auto issue_w = [&](int s) {  // this wave's rows of local stage s (clamped) into slot s % WR
-      const int sg_ = s0 + min(s, last);
-#pragma unroll
-      for (int i = 0; i < WINS; i++)
-        if (64 * i + lane < WSLOTS)
-          dma16(wsrc[i] + gemm_chunk_off<FMT>(sg_, wc[i]), &Wg[pw][s % WR][1024 * i]);
-    };
-    // Dequantize local stage s of this wave's rows: task t = 4 rr + 2 h + qq
-    // (row rr, half h of the 64 elements, 16-element quarter qq of the half),
-    // t = lane + 64 round.
-    auto dequant = [&](int s) {
-      const int j = (s0 + s) & 3;  // group of the unit (Q4_K scale pick)
-      const uint8_t *wg = Wg[pw][s % WR];
-      uint4 hd[3], qs[3], qh[3];
-      {
-        uint32_t ad[3 * 3];
-#pragma unroll
-        for (int round = 0; round < 3; round++) {
-          const int t = min(lane + 64 * round, R::TASKS - 1);
-          const int rr = t >> 2, qq = t & 1;
-          ad[3 * round] = (uint32_t)(uintptr_t)(lds_void_t *)(wg + 16 * C * rr);
-          ad[3 * round + 1] = (uint32_t)(uintptr_t)(lds_void_t *)(wg + 16 * C * rr + 16 + 16 * qq);
-          ad[3 * round + 2] = (uint32_t)(uintptr_t)(lds_void_t *)(wg + 16 * C * rr + 48);
-        }
-        if constexpr (FMT == T_Q4_K) {
-          if constexpr (R::ROUNDS == 3) {
-            const uint32_t a6[6] = {ad[0], ad[1], ad[3], ad[4], ad[6], ad[7]};
-            uint4 v[6];
-            lds_read6(a6, v);
-            hd[0] = v[0]; qs[0] = v[1]; hd[1] = v[2]; qs[1] = v[3]; hd[2] = v[4]; qs[2] = v[5];
-          } else {
-            const uint32_t a4[4] = {ad[0], ad[1], ad[3], ad[4]};
-            uint4 v[4];
-            lds_read4(a4, v);
-            hd[0] = v[0]; qs[0] = v[1]; hd[1] = v[2]; qs[1] = v[3];
-          }
-        } else {
-          if constexpr (R::ROUNDS == 3) {
-            const uint32_t a6[6] = {ad[0], ad[1], ad[2], ad[3], ad[4], ad[5]};
-            uint4 v[6];
-            lds_read6(a6, v);
-            hd[0] = v[0]; qs[0] = v[1]; qh[0] = v[2]; hd[1] = v[3]; qs[1] = v[4]; qh[1] = v[5];
-            const uint32_t a2[2] = {ad[6], ad[7]};
-            uint4 w[2];
-            lds_read2_a(a2, w);
-            hd[2] = w[0]; qs[2] = w[1];
-            const uint32_t a1[2] = {ad[8], ad[8]};
-            lds_read2_a(a1, w);
-            qh[2] = w[0];
-          } else {
-            const uint32_t a6[6] = {ad[0], ad[1], ad[2], ad[3], ad[4], ad[5]};
-            uint4 v[6];
-            lds_read6(a6, v);
-            hd[0] = v[0]; qs[0] = v[1]; qh[0] = v[2]; hd[1] = v[3]; qs[1] = v[4]; qh[1] = v[5];
-          }
-        }
-      }
-#pragma unroll
-      for (int round = 0; round < R::ROUNDS; round++) {
-        const int t = lane + 64 * round;
-        if (round < R::ROUNDS - 1 || t < R::TASKS) {
-          const int rr = t >> 2, h = (t >> 1) & 1, qq = t & 1;
-          const int r = PROWS * pw + rr;
-          const bool ok = m0 + r < rows;
-          const uint32_t qw[4] = {qs[round].x, qs[round].y, qs[round].z, qs[round].w};
-          const uint32_t sh = 4u * (uint32_t)h;
-          uint32_t o[8];
-          if constexpr (FMT == T_Q4_K) {
-            uint32_t sc, mn;
-            scale_min_k4_sel(2 * j + h, hd[round].y, hd[round].z, hd[round].w, sc, mn);
-            const float ds = ok ? h2f(hd[round].x) * (float)sc : 0.f;
-            const float nm = ok ? -(h2f(hd[round].x >> 16) * (float)mn) : 0.f;
-#pragma unroll
-            for (int i = 0; i < 4; i++) {
-              const uint32_t qv = (qw[i] >> sh) & 0x0F0F0F0Fu;
-              o[2 * i] = pack_bf16(fmaf(ds, cvt_ubyte<0>(qv), nm), fmaf(ds, cvt_ubyte<1>(qv), nm));
-              o[2 * i + 1] = pack_bf16(fmaf(ds, cvt_ubyte<2>(qv), nm), fmaf(ds, cvt_ubyte<3>(qv), nm));
-            }
-          } else {
-            // dequant_q6_k: (d * sc) * (q - 32), one rounding: fma(ds, q, -32 ds)
-            const int g = 2 * h + qq;
-            const int sc8 = (int)(int8_t)(hd[round].x >> (8 * g));
-            const float ds = ok ? h2f(hd[round].y) * (float)sc8 : 0.f;
-            const float nm = -32.0f * ds;
-            const uint32_t hw = g == 0 ? qh[round].x : g == 1 ? qh[round].y : g == 2 ? qh[round].z : qh[round].w;
-#pragma unroll
-            for (int i = 0; i < 4; i++) {
-              const uint32_t b2 = (hw >> (8 * i)) & 0xFFu;
-              const uint32_t hi = (b2 | (b2 << 6) | (b2 << 12) | (b2 << 18)) & 0x03030303u;
-              const uint32_t qv = ((qw[i] >> sh) & 0x0F0F0F0Fu) | (hi << 4);
-              o[2 * i] = pack_bf16(fmaf(ds, cvt_ubyte<0>(qv), nm), fmaf(ds, cvt_ubyte<1>(qv), nm));
-              o[2 * i + 1] = pack_bf16(fmaf(ds, cvt_ubyte<2>(qv), nm), fmaf(ds, cvt_ubyte<3>(qv), nm));
-            }
-          }
-          uint16_t *dst = &As[s & 1][((h * AT_ + (r >> 4)) * 64 + (r & 15) + 32 * qq) * 8];
-          *(uint4 *)dst = make_uint4(o[0], o[1], o[2], o[3]);
-          *(uint4 *)(dst + 128) = make_uint4(o[4], o[5], o[6], o[7]);
-        }
-      }
-    };
-    if constexpr (NXR == 3) {
-      // prologue: stages 0 and 1 in flight, stage 0 dequantized
-      issue_x(0);
-      issue_w(0);
-      issue_x(1);
-      issue_w(1);
-      wait_vm<XPW + WINS>();
-      dequant(0);
-      wait_lgkm0();
-      __builtin_amdgcn_s_barrier();
-      for (int kt = 0; kt < stages; kt++) {
-        issue_x(kt + 2);
-        issue_w(kt + 2);
-        wait_vm<XPW + WINS>();  // stage kt + 1 (X and this wave's W rows) in LDS
-        if (kt + 1 < stages) dequant(kt + 1);
-        wait_lgkm0();
-        __builtin_amdgcn_s_barrier();
-      }
-    } else {
-      static_assert(NXR == 2, "2 or 3 X slots");
-      issue_x(0);
-      issue_w(0);
-      issue_w(1);
-      wait_vm<WINS>();  // X and W of stage 0
-      dequant(0);
-      wait_lgkm0();
-      __builtin_amdgcn_s_barrier();
-      for (int kt = 0; kt < stages; kt++) {
-        issue_x(kt + 1);
-        issue_w(kt + 2);
-        wait_vm<XPW + WINS>();  // W of stage kt + 1
-        if (kt + 1 < stages) dequant(kt + 1);
-        wait_vm<WINS>();  // X of stage kt + 1
-        wait_lgkm0();
-        __builtin_amdgcn_s_barrier();
-      }
-    }
-    wait_vm<0>();  // drain the clamped loads before the block ends
-    return;
-  }
-
-  // ---- multiply waves
-  const int wm = wave % R::WGM, wn = wave / R::WGM;
-  f32x4_t acc[TM][TN];
-#pragma unroll
-  for (int i = 0; i < TM; i++)
-#pragma unroll
-    for (int jj = 0; jj < TN; jj++) acc[i][jj] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-  __builtin_amdgcn_s_barrier();  // stage 0 in LDS
-  for (int kt = 0; kt < stages; kt++) {
-    const uint16_t *A = As[kt & 1], *B = Xs[kt % NXR];
-#pragma unroll
-    for (int ks = 0; ks < 2; ks++) {
-      bf16x8_t av[TM];
-#pragma unroll
-      for (int i = 0; i < TM; i++)
-        av[i] = *(const bf16x8_t *)(A + ((ks * AT_ + TM * wm + i) * 64 + lane) * 8);
-#pragma unroll
-      for (int jn = 0; jn < TN; jn++) {
-        const bf16x8_t bb = *(const bf16x8_t *)(B + ((ks * BT_ + TN * wn + jn) * 64 + lane) * 8);
-#pragma unroll
-        for (int i = 0; i < TM; i++)
-          acc[i][jn] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(av[i], bb, acc[i][jn], 0, 0, 0);
-      }
-    }
-    wait_lgkm0();
-    __builtin_amdgcn_s_barrier();
-  }
-  // D layout: lane holds rows 4*(lane/16)+r (weight rows) of column lane%16 (token).
-  float *Y = a.ksplit > 1 ? sg.part + (long)split * a.n * rows : sg.y;
-#pragma unroll
-  for (int i = 0; i < TM; i++) {
-    const int m = m0 + WM * wm + 16 * i + 4 * (lane >> 4);
-#pragma unroll
-    for (int jj = 0; jj < TN; jj++) {
-      const int t = n0 + WN * wn + 16 * jj + (lane & 15);
-      if (t >= a.n) continue;
-      float *yp = Y + (long)t * rows + m;
-      if (m + 3 < rows && (rows & 3) == 0) {
-        *(float4 *)yp = make_float4(acc[i][jj][0], acc[i][jj][1], acc[i][jj][2], acc[i][jj][3]);
-      } else {
-#pragma unroll
-        for (int r = 0; r < 4; r++)
-          if (m + r < rows) yp[r] = acc[i][jj][r];
-      }
-    }
-  }
-}
-
 // ----------------------------------------------------------- bf16 kernel, direct X
 // Block tile 160 rows x 256 tokens, 512 threads, K-steps ("stages") of 64.
 // Waves 0-3 multiply: wave w owns all 160 rows x tokens 64w .. 64w + 63 of
@@ -644,12 +263,16 @@ __global__ __launch_bounds__(512) void k_gemm_bf16_ring(GemmArgs a) {
 // fragment order by a pre-pass) from global memory (L2) straight into
 // registers, one stage ahead.  The only LDS operand is the dequantized W
 // tile (fragment-major, two slots), read once per 4 MFMAs.  Waves 4-7
-// produce it as in the ring kernel: each fetches its 40 rows' stage records
-// two stages ahead into a ring private to the wave (straight to LDS) and
-// dequantizes them to bf16.  One barrier per stage.
-// LDS traffic per stage: 20 KiB of A written, 4 x 20 KiB read (the ring
-// kernel also moved 2 x 64 KiB of X); load path per stage: 32 KiB of X plus
-// the W records.
+// produce it: each fetches, two stages ahead, the stage records of its own 40
+// rows into a ring private to the wave (straight to LDS: a producer waits only
+// for its own loads) and dequantizes them (Q4_K: d*sc*q - dmin*m; Q6_K:
+// d*sc*(q - 32); rounded to bf16, RNE).  One barrier per stage.
+// LDS traffic per stage: 20 KiB of A written, 4 x 20 KiB read; load path per
+// stage: 32 KiB of X plus the W records.
+// Blocks: (row tile, token tile, K split).  A launch covers up to
+// GEMM_MAX_SEG matrices sharing the input (row tiles numbered across them);
+// with ksplit > 1 a block covers stages [S*s/ksplit, S*(s+1)/ksplit) and
+// writes a partial product, which k_gemm_reduce sums in a fixed order.
 template <int FMT>
 struct Direct {
   static constexpr int TBM = 160, TBN = 256;
@@ -899,7 +522,7 @@ __global__ __launch_bounds__(512) void k_gemm_bf16_direct(GemmArgs a) {
     }
     return;
   }
-  float *Y = a.ksplit > 1 ? sg.part + (long)split * a.n * rows : sg.y;
+  float *Y = sg.part ? sg.part + (long)split * a.n * rows : sg.y;
 #pragma unroll
   for (int i = 0; i < AT_; i++) {
     const int m = m0 + 16 * i + 4 * (lane >> 4);
@@ -1387,33 +1010,67 @@ int gemm_ksplit(int tiles, int stages, int num_cus) {
   return best;
 }
 
+// K split of the short-batch kernel's launch of `tiles` row tiles and Tq
+// quads per row: the least estimated time, in units of one quad's work of a
+// block (one block per CU; about 4.8 us for Q6_K at 16 tokens): half a unit
+// to start, and a reduction launch when K is split.  Measured, us a call: 3584 x
+// 18944 Q6_K at 37 tokens (32 tiles) 107 unsplit, 50 in 3, 36 in 5, 32 in 8, 41
+// in 10 (a second round); 18944 x 3584 Q4_K (170 tiles) 28 unsplit, 35 in 2;
+// 8192 x 2048 Q8_0 at 8 tokens (74 tiles) 15.8 unsplit, 14.5 in 2.
+int gemm_quad_ksplit(int tiles, int Tq, int num_cus) {
+  int best = 1;
+  double best_t = 1e30;
+  for (int ks = 1; ks <= std::min(Tq, 16); ks++) {
+    const int rounds = (tiles * ks + num_cus - 1) / num_cus;
+    const double t = rounds * (0.5 + (Tq + ks - 1) / ks) + (ks > 1 ? 0.7 + 0.05 * ks : 0.0);
+    if (t < best_t - 1e-9) {
+      best_t = t;
+      best = ks;
+    }
+  }
+  return best;
+}
+
 namespace {
 struct GemmPlan {
-  bool direct;
+  bool quad;                        // gq_gemm_quad.hip's kernel
   int tbm, tbn, ntiles, tiles, ksplit;
 };
-// Kernel choice: the direct-X kernel (160 x 256 tiles, X fragments loaded
-// straight into the multiply waves' registers) for batches longer than 128
-// tokens; the ring kernel (160 x 256 tiles, X through LDS) for shorter ones.
-GemmPlan gemm_plan(const gq_weight *const *ws, int count, int n, int num_cus, bool add) {
+GemmPlan gemm_plan(const gq_weight *const *ws, int count, int n, int num_cus) {
   GemmPlan p;
-  p.direct = n > 128;
-  p.tbm = BM;
-  p.tbn = BN;
+  p.quad = gemm_uses_quad(ws, count, n);
+  p.tbm = p.quad ? GEMM_QUAD_ROWS : BM;
+  p.tbn = p.quad ? 16 * gemm_quad_nt(n) : BN;
   p.ntiles = (n + p.tbn - 1) / p.tbn;
   int mt = 0;
   for (int i = 0; i < count; i++) mt += (ws[i]->L.rows + p.tbm - 1) / p.tbm;
   p.tiles = mt * p.ntiles;
-  p.ksplit = gemm_ksplit(p.tiles, ws[0]->L.units * 4, num_cus);
-  // an accumulating launch adds its product in gemm_reduce
-  if (add && p.ksplit == 1) p.ksplit = ws[0]->L.units * 4 >= 2 ? 2 : 1;
+  const int U = ws[0]->L.units, parts = p.quad ? (U + 3) / 4 : U * 4;
+  p.ksplit = p.quad ? gemm_quad_ksplit(p.tiles, parts, num_cus) : gemm_ksplit(p.tiles, parts, num_cus);
   return p;
 }
 }  // namespace
 
+// Batches of up to 128 tokens (the largest whose accumulators and X fragments
+// fit a wave's registers), on weights in the quad layout (all dense ones; not
+// stacked experts of other than 16 m rows).  Measured at 128 tokens against
+// the 160 x 256 kernel at 160 (one token tile either way), us a call: 3584 x
+// 18944 Q6_K 47 against 70, 18944 x 3584 Q4_K 44 against 51.
+bool gemm_uses_quad(const gq_weight *const *ws, int count, int n) {
+  for (int i = 0; i < count; i++)
+    if (!ws[i]->L.quad) return false;
+  return n <= GEMM_QUAD_MAX;
+}
+
+// bf16 of X in fragment form for a batch of n (quad: gemm_uses_quad).
+size_t gemm_x_elems(int units, int n, bool quad) {
+  if (quad) return (size_t)16 * gemm_quad_nt(n) * ((units + 3) / 4) * 1024;
+  return (size_t)((n + GEMM_NPAD - 1) / GEMM_NPAD * GEMM_NPAD) * units * 256;
+}
+
 size_t gemm_part_floats(const gq_weight *const *ws, int count, int n, int num_cus, bool add) {
-  const GemmPlan p = gemm_plan(ws, count, n, num_cus, add);
-  if (p.ksplit == 1) return 0;
+  const GemmPlan p = gemm_plan(ws, count, n, num_cus);
+  if (p.ksplit == 1 && !add) return 0;
   size_t rows = 0;
   for (int i = 0; i < count; i++) rows += (size_t)ws[i]->L.rows;
   return (size_t)p.ksplit * n * rows;
@@ -1424,7 +1081,7 @@ size_t gemm_workspace_bytes(const gq_weight *w, int n, int mode, int num_cus) {
   if (mode == GQ_GEMM_BF16) {
     if (w->L.dtype != T_Q4_K && w->L.dtype != T_Q6_K && w->L.dtype != T_Q5_K && w->L.dtype != T_Q8_0)
       return (size_t)-1;
-    const size_t xb = (size_t)((n + GEMM_NPAD - 1) / GEMM_NPAD * GEMM_NPAD) * kpad * 2;
+    const size_t xb = gemm_x_elems(w->L.units, n, gemm_uses_quad(&w, 1, n)) * 2;
     return ((xb + 255) & ~(size_t)255) + gemm_part_floats(&w, 1, n, num_cus, false) * 4 + 256;
   }
   if (w->L.dtype != T_Q4_K && w->L.dtype != T_Q6_K) return (size_t)-1;
@@ -1447,10 +1104,10 @@ hipError_t launch_gemm_bf16(const gq_weight *const *ws, float *const *ys, int co
                             hipStream_t st, int *defer) {
   if (count < 1 || count > GEMM_MAX_SEG || n <= 0) return hipErrorInvalidValue;
   const int fmt = ws[0]->L.dtype;
-  const GemmPlan p = gemm_plan(ws, count, n, num_cus, add);
+  const GemmPlan p = gemm_plan(ws, count, n, num_cus);
+  const bool parts = add || p.ksplit > 1;  // partial products, summed by k_gemm_reduce
   GemmArgs a{};
   a.nseg = count;
-  a.ntiles = p.ntiles;
   a.ksplit = p.ksplit;
   a.n = n;
   a.kpad = ws[0]->L.units * 256;
@@ -1458,31 +1115,36 @@ hipError_t launch_gemm_bf16(const gq_weight *const *ws, float *const *ys, int co
   int tb = 0;
   size_t po = 0;
   for (int i = 0; i < count; i++) {
-    if (ws[i]->L.dtype != fmt || ws[i]->L.units != ws[0]->L.units || !ws[i]->gemm_raw)
+    if (ws[i]->L.dtype != fmt || ws[i]->L.units != ws[0]->L.units || !(p.quad || ws[i]->gemm_raw))
       return hipErrorInvalidValue;
     a.seg[i].rec = ws[i]->gemm_raw;
+    a.seg[i].body = ws[i]->body;
+    a.seg[i].d = ws[i]->d;
     a.seg[i].y = ys[i];
     a.seg[i].rows = ws[i]->L.rows;
     a.seg[i].tile_begin = tb;
-    a.seg[i].part = p.ksplit > 1 ? part + po : nullptr;
+    a.seg[i].part = parts ? part + po : nullptr;
     tb += (ws[i]->L.rows + p.tbm - 1) / p.tbm;
     po += (size_t)p.ksplit * n * ws[i]->L.rows;
   }
-  if (p.ksplit > 1 && !part) return hipErrorInvalidValue;
+  if (parts && !part) return hipErrorInvalidValue;
+  a.ntiles = p.quad ? tb : p.ntiles;
   const long nb = (long)tb * p.ntiles * p.ksplit;
   if (nb > 0x7fffffffL) return hipErrorInvalidValue;
-  void (*kern)(GemmArgs);
-  // Q5_K and Q8_0 run the direct kernel at every batch size (the ring
-  // kernel's LDS has no room for Q8_0's five-chunk records)
-  if (fmt == T_Q5_K) kern = k_gemm_bf16_direct<T_Q5_K>;
-  else if (fmt == T_Q8_0) kern = k_gemm_bf16_direct<T_Q8_0>;
-  else if (p.direct) kern = fmt == T_Q4_K ? k_gemm_bf16_direct<T_Q4_K> : k_gemm_bf16_direct<T_Q6_K>;
-  else if (fmt == T_Q4_K) kern = k_gemm_bf16_ring<160, 256, 3, T_Q4_K>;
-  else if (fmt == T_Q6_K) kern = k_gemm_bf16_ring<160, 256, 3, T_Q6_K>;
-  else return hipErrorInvalidValue;
-  hipLaunchKernelGGL(kern, dim3((unsigned)nb), dim3(512), 0, st, a);
-  hipError_t e = hipGetLastError();
-  if (e != hipSuccess || p.ksplit == 1) return e;
+  hipError_t e;
+  if (p.quad) {
+    e = launch_gemm_quad(a, fmt, (int)nb, st);
+  } else {
+    void (*kern)(GemmArgs);
+    if (fmt == T_Q5_K) kern = k_gemm_bf16_direct<T_Q5_K>;
+    else if (fmt == T_Q8_0) kern = k_gemm_bf16_direct<T_Q8_0>;
+    else if (fmt == T_Q4_K) kern = k_gemm_bf16_direct<T_Q4_K>;
+    else if (fmt == T_Q6_K) kern = k_gemm_bf16_direct<T_Q6_K>;
+    else return hipErrorInvalidValue;
+    hipLaunchKernelGGL(kern, dim3((unsigned)nb), dim3(512), 0, st, a);
+    e = hipGetLastError();
+  }
+  if (e != hipSuccess || !parts) return e;
   if (defer && add) {
     *defer = p.ksplit;
     return hipSuccess;
@@ -1505,7 +1167,7 @@ hipError_t launch_gemm_bf16(const gq_weight *const *ws, float *const *ys, int co
 hipError_t launch_gemm_bf16_swiglu(const gq_weight *gate, const gq_weight *up, const uint16_t *xb, int n,
                                    uint16_t *hb, int num_cus, hipStream_t st) {
   (void)num_cus;
-  if (n <= 128) return hipErrorNotSupported;  // the ring kernel's batches
+  if (n <= GEMM_QUAD_MAX) return hipErrorNotSupported;  // the short-batch kernel's
   const Layout &L = gate->L;
   if (up->L.dtype != L.dtype || up->L.units != L.units || up->L.rows != L.rows || !gate->gemm_raw ||
       !up->gemm_raw)
@@ -1546,9 +1208,10 @@ hipError_t launch_gemm(const gq_weight *w, const float *X, int n, float *Y, int 
   const int kpad = L.units * 256;
   if (mode == GQ_GEMM_BF16) {
     uint16_t *xb = (uint16_t *)workspace;
-    const size_t xbb = (size_t)((n + GEMM_NPAD - 1) / GEMM_NPAD * GEMM_NPAD) * kpad * 2;
+    const bool quad = gemm_uses_quad(&w, 1, n);
+    const size_t xbb = gemm_x_elems(L.units, n, quad) * 2;
     float *part = (float *)((char *)workspace + ((xbb + 255) & ~(size_t)255));
-    hipError_t e = launch_x_to_frag(X, n, L.k, xb, st);
+    hipError_t e = quad ? launch_x_to_quad(X, n, L.k, xb, st) : launch_x_to_frag(X, n, L.k, xb, st);
     if (e != hipSuccess) return e;
     return launch_gemm_bf16(&w, &Y, 1, xb, n, part, false, num_cus, st);
   } else {

@@ -223,16 +223,21 @@ hipError_t launch_gemm_records(const gq_weight *w, uint8_t *out, hipStream_t st)
 // split the partial products part [ksplit][n][rows].
 constexpr int GEMM_MAX_SEG = 3;
 struct GemmSeg {
-  const uint8_t *rec;  // stage records
+  const uint8_t *rec;   // stage records (direct kernel)
+  const uint8_t *body;  // quad-layout body and d array (short-batch kernel)
+  const uint16_t *d;
   float *y;
-  float *part;
+  float *part;          // if set, the partial products go here instead of to y
   int rows;
   int tile_begin;      // first row tile of this matrix in the launch
 };
 struct GemmArgs {
   GemmSeg seg[GEMM_MAX_SEG];
   int nseg, ntiles, ksplit, n, kpad;
-  const uint16_t *xb;  // X as bf16 MFMA fragments [npad/16][kpad/32][64 lanes][8]
+  // X as bf16 MFMA fragments: [npad/16][kpad/32][64 lanes][8], or for the
+  // short-batch kernel (whose ntiles is the number of row tiles)
+  // [npad/16][quads][32 steps][64 lanes][8]
+  const uint16_t *xb;
   // pair (direct kernel, no K split): seg[0] = gate, seg[1] = up of one
   // shape; a block tile holds 80 rows of each, and the epilogue writes
   // silu(gate . x) * (up . x) as bf16 fragments hb (the next GEMM's X, hkpad
@@ -240,14 +245,23 @@ struct GemmArgs {
   int pair, hkpad;
   uint16_t *hb;
 };
-// X fragments must cover n rounded up to GEMM_NPAD (a multiple of the
+// Batches of up to GEMM_QUAD_MAX tokens run on the quad-layout weights
+// (gq_gemm_quad.hip), whose X fragments cover 16 * gemm_quad_nt(n) tokens;
+// for longer ones X fragments must cover n rounded up to GEMM_NPAD (the
 // 256-token tile).
-constexpr int GEMM_NPAD = 512;
+constexpr int GEMM_NPAD = 256;
+constexpr int GEMM_QUAD_MAX = 128;
+constexpr int GEMM_QUAD_ROWS = 112;  // weight rows per block of that kernel
+bool gemm_uses_quad(const gq_weight *const *ws, int count, int n);
+int gemm_quad_nt(int n);
+size_t gemm_x_elems(int units, int n, bool quad);
+hipError_t launch_x_to_quad(const float *X, int n, int k, uint16_t *xb, hipStream_t st);
+hipError_t launch_gemm_quad(const GemmArgs &a, int fmt, int blocks, hipStream_t st);
 // K split of a launch with this many row x token tiles and stages.
 int gemm_ksplit(int tiles, int stages, int num_cus);
-// Y_i (+)= W_i . X for count <= GEMM_MAX_SEG weights of one dtype (Q4_K or
-// Q6_K) and in_dim, on X already in fragment form (xb, n tokens).  add: Y_i
-// += (else =; an accumulating launch always splits K and adds in the
+// Y_i (+)= W_i . X for count <= GEMM_MAX_SEG weights of one dtype and in_dim,
+// on X already in fragment form (xb, n tokens; the form gemm_uses_quad tells).
+// add: Y_i += (else =; an accumulating launch writes partials and adds in the
 // reduction).  part: gemm_part_floats floats.
 // defer (accumulating launches only): the reduction is left to the
 // caller; *defer receives the K split whose partials part holds.
@@ -257,7 +271,7 @@ hipError_t launch_gemm_bf16(const gq_weight *const *ws, float *const *ys, int co
 // The gate/up pair of the SwiGLU on the direct kernel: hb = bf16 fragments
 // of silu(gate . X) * (up . X) ([npad/16][round_up(F, 256)/32][64][8], the
 // next GEMM's X; zero past n and F).  hipErrorNotSupported when the batch
-// takes the ring kernel (n <= 128) or the two differ in type or shape: the
+// takes the short-batch kernel (n <= 128) or the two differ in type or shape: the
 // caller then runs launch_gemm_bf16 and its own SwiGLU.
 hipError_t launch_gemm_bf16_swiglu(const gq_weight *gate, const gq_weight *up, const uint16_t *xb, int n,
                                    uint16_t *hb, int num_cus, hipStream_t st);

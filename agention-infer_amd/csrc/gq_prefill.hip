@@ -34,9 +34,13 @@ __device__ __forceinline__ uint32_t bf16_bits(float f) {
 }
 
 // Position of elements (t, c .. c + 7) (c % 8 == 0) in the GEMM's X
-// fragments: fragment (t / 16, c / 32) of 64 lanes x 8 bf16, lane
-// t % 16 + 16 * ((c % 32) / 8).
-__device__ __forceinline__ long frag_slot(int t, int c, int ksteps) {
+// fragments of 64 lanes x 8 bf16: fragment (t / 16, c / 32), lane
+// t % 16 + 16 * ((c % 32) / 8), or for a short batch (quad) fragment
+// (t / 16, c / 1024, step (c % 256) / 8), lane t % 16 + 16 * (unit of the
+// quad).  ksteps: fragments per token tile.
+__device__ __forceinline__ long frag_slot(int t, int c, int ksteps, bool quad) {
+  if (quad)
+    return (((long)(t >> 4) * ksteps + 32 * (c >> 10) + ((c & 255) >> 3)) * 64 + (t & 15) + 16 * ((c >> 8) & 3)) * 8;
   return (((long)(t >> 4) * ksteps + (c >> 5)) * 64 + (t & 15) + 16 * ((c & 31) >> 3)) * 8;
 }
 
@@ -76,7 +80,7 @@ constexpr int NORM_GROUPS = 4;
 // part[1][t] + ... (in that order, as k_gemm_reduce) is done here, and the
 // new row is stored back to x.
 __global__ __launch_bounds__(256) void k_norm_to_frag(float *__restrict__ x, const float *__restrict__ w, int n,
-                                                      int H, int kpad, float eps, uint16_t *__restrict__ xb,
+                                                      int H, int kpad, bool quad, float eps, uint16_t *__restrict__ xb,
                                                       const float *__restrict__ part, int ksplit) {
   __shared__ float red[4];
   const int t = blockIdx.x, ksteps = kpad / 32;
@@ -138,7 +142,7 @@ __global__ __launch_bounds__(256) void k_norm_to_frag(float *__restrict__ x, con
 #pragma unroll
       for (int e = 0; e < 8; e++) o[e] = 0.f;
     }
-    put_frag8(xb, frag_slot(t, c, ksteps), o);
+    put_frag8(xb, frag_slot(t, c, ksteps, quad), o);
   }
 }
 
@@ -147,7 +151,7 @@ __global__ __launch_bounds__(256) void k_norm_to_frag(float *__restrict__ x, con
 // fragment (16 tokens x 32 columns, 1 KiB contiguous): lane l converts
 // token 16 nt + l % 16, columns 32 ks + 8 (l / 16) .. + 8.
 __global__ __launch_bounds__(256) void k_swiglu_to_frag(const float *g, const float *u, int n, int F,
-                                                        int npad, int kpad, uint16_t *xb) {
+                                                        int npad, int kpad, bool quad, uint16_t *xb) {
   const int ksteps = kpad / 32, lane = threadIdx.x & 63;
   const long f = (long)blockIdx.x * 4 + (threadIdx.x >> 6);
   if (f >= (long)(npad / 16) * ksteps) return;
@@ -166,7 +170,7 @@ __global__ __launch_bounds__(256) void k_swiglu_to_frag(const float *g, const fl
 #pragma unroll
     for (int e = 0; e < 8; e++) v[e] = 0.f;
   }
-  put_frag8(xb, frag_slot(t, c, ksteps), v);
+  put_frag8(xb, frag_slot(t, c, ksteps, quad), v);
 }
 
 // NEOX RoPE (cpu_path.rs:99-133, angle pos / theta^(2i/hd)) of q [n][nh*hd]
@@ -357,7 +361,7 @@ __device__ __forceinline__ uint32_t kv_slot(int row, int blk) {
 template <int HD>
 __global__ __launch_bounds__(512) void k_attn_prefill(const float *q, const uint16_t *kc,
                                                       const uint16_t *vc, int pos0, int n, int nh,
-                                                      int group, uint16_t *xb) {
+                                                      int group, int kpad, bool quad, uint16_t *xb) {
   constexpr int KS = HD / 32, DT = HD / 16;
   constexpr int NB = HD / 8;                 // 16-byte blocks per K/V row
   constexpr int TILE = 64 * HD * 2;          // bytes of one K or V tile
@@ -557,7 +561,7 @@ __global__ __launch_bounds__(512) void k_attn_prefill(const float *q, const uint
     const float M = fmaxf(mrow, m1);  // mrow is finite: chunk 0 is in this half
     const float f0 = exp2f(mrow - M), f1 = m1 == -INFINITY ? 0.f : exp2f(m1 - M);
     const float L = lrow * f0 + l1 * f1;
-    const int ksteps = nh * HD / 32;
+    const int ksteps = kpad / 32;
 #pragma unroll
     for (int d = 0; d < DT; d++) {
       float v[8];
@@ -569,7 +573,11 @@ __global__ __launch_bounds__(512) void k_attn_prefill(const float *q, const uint
         v[4 + i] = __uint_as_float(r[1]);  // the odd group's
       }
       if (((lane >> 4) & 1) == 0 && tq < n)
-        put_frag8(xb, frag_slot(tq, h * HD + 16 * d + 8 * (lane >> 5), ksteps), v);
+        put_frag8(xb, frag_slot(tq, h * HD + 16 * d + 8 * (lane >> 5), ksteps, quad), v);
+    }
+    if (h == nh - 1 && tq < n) {  // the columns' padding (the weights are zero there, X must be finite)
+      const float z[8] = {};
+      for (int c = nh * HD + 8 * (lane >> 4); c < kpad; c += 32) put_frag8(xb, frag_slot(tq, c, ksteps, quad), z);
     }
   }
 }
@@ -577,24 +585,27 @@ __global__ __launch_bounds__(512) void k_attn_prefill(const float *q, const uint
 // ------------------------------------------------------------------ host
 static int round_up(int v, int m) { return (v + m - 1) / m * m; }
 
-// The largest K-split partial buffer of any launch of a pass of up to nmax
-// tokens.  Passes of up to 256 tokens use taller row tiles (fewer tiles, a
-// larger split), so both tile regimes are sized at their largest batch.
+// The largest partial buffer of any launch of a pass of up to nmax tokens
+// (the K split depends on the batch's tiles, of 16 tokens for a short batch).
 size_t prefill_part_floats(const DecodeLaunch &m, int nmax, int num_cus) {
   size_t best = 0;
-  for (int nn : {std::min(nmax, 256), nmax})
-  for (int L = 0; L < m.n_layers; L++) {
-    const int nmax = nn;
-    const gq_weight *qkv[3] = {m.wq[L], m.wk[L], m.wv[L]};
-    for (int i = 0; i < 3; i++) best = std::max(best, gemm_part_floats(&qkv[i], 1, nmax, num_cus, false));
-    if (qkv[0]->L.dtype == qkv[1]->L.dtype && qkv[1]->L.dtype == qkv[2]->L.dtype)
-      best = std::max(best, gemm_part_floats(qkv, 3, nmax, num_cus, false));
-    best = std::max(best, gemm_part_floats(&m.wo[L], 1, nmax, num_cus, true));
-    const gq_weight *gu[2] = {m.wgate[L], m.wup[L]};
-    best = std::max(best, gemm_part_floats(gu, 2, nmax, num_cus, false));
-    best = std::max(best, gemm_part_floats(&m.wdown[L], 1, nmax, num_cus, true));
+  for (int n = 16;; n = std::min(n + 16, nmax)) {
+    for (int L = 0; L < m.n_layers; L++) {
+      const gq_weight *qkv[3] = {m.wq[L], m.wk[L], m.wv[L]};
+      for (int set = 1; set < 8; set++) {  // whichever of them share a type and so a launch
+        const gq_weight *grp[3];
+        int c = 0;
+        for (int i = 0; i < 3; i++)
+          if (set >> i & 1) grp[c++] = qkv[i];
+        best = std::max(best, gemm_part_floats(grp, c, n, num_cus, false));
+      }
+      best = std::max(best, gemm_part_floats(&m.wo[L], 1, n, num_cus, true));
+      const gq_weight *gu[2] = {m.wgate[L], m.wup[L]};
+      best = std::max(best, gemm_part_floats(gu, 2, n, num_cus, false));
+      best = std::max(best, gemm_part_floats(&m.wdown[L], 1, n, num_cus, true));
+    }
+    if (n >= nmax) return best;
   }
-  return best;
 }
 
 // One pass of n <= PREFILL_MAX tokens (tokens_dev) at positions pos0 ..
@@ -604,13 +615,14 @@ hipError_t launch_prefill(const DecodeLaunch &m, const PrefillBufs &b, const int
   if (n < 1 || n > PREFILL_MAX) return hipErrorInvalidValue;
   const int H = m.hidden, hd = m.head_dim, nh = m.n_heads, nkv = m.n_kv_heads;
   const int kvd = nkv * hd, qd = nh * hd, F = m.ffn, group = nh / nkv;
-  const int npad = round_up(n, GEMM_NPAD);
+  const bool quad = n <= GEMM_QUAD_MAX;  // (a decoder's weights are all in the quad layout)
+  const int npad = quad ? 16 * gemm_quad_nt(n) : round_up(n, GEMM_NPAD), kq = quad ? 1024 : 256;
   hipError_t e;
   hipLaunchKernelGGL(k_embed_rows, dim3(n), dim3(256), 0, s, m.embd, tokens_dev, H, b.x);
   int pending = 0;  // K split of partials left for the next norm to add into x
   for (int L = 0; L < m.n_layers; L++) {
     hipLaunchKernelGGL(k_norm_to_frag, dim3(npad), dim3(256), 0, s, b.x, m.attn_norm[L], n, H,
-                       round_up(H, 256), m.eps, b.xb, b.part, pending);
+                       round_up(H, kq), quad, m.eps, b.xb, b.part, pending);
     pending = 0;
     // q, k, v: one launch per distinct dtype (attn_v is Q6_K in some files)
     const gq_weight *qkv[3] = {m.wq[L], m.wk[L], m.wv[L]};
@@ -652,18 +664,20 @@ hipError_t launch_prefill(const DecodeLaunch &m, const PrefillBufs &b, const int
     const int items = (n + PF_Q - 1) / PF_Q * nkv;  // (query tile, KV head)
     const dim3 ag(8 * group * ((items + 7) / 8));
     if (hd == 128)
-      hipLaunchKernelGGL(k_attn_prefill<128>, ag, dim3(512), 0, s, b.q, kc, vc, pos0, n, nh, group, b.xb);
+      hipLaunchKernelGGL(k_attn_prefill<128>, ag, dim3(512), 0, s, b.q, kc, vc, pos0, n, nh, group,
+                         round_up(qd, kq), quad, b.xb);
     else
-      hipLaunchKernelGGL(k_attn_prefill<64>, ag, dim3(512), 0, s, b.q, kc, vc, pos0, n, nh, group, b.xb);
+      hipLaunchKernelGGL(k_attn_prefill<64>, ag, dim3(512), 0, s, b.q, kc, vc, pos0, n, nh, group,
+                         round_up(qd, kq), quad, b.xb);
     float *xo[1] = {b.x};
     if ((e = launch_gemm_bf16(&m.wo[L], xo, 1, b.xb, n, b.part, true, num_cus, s, &pending)) != hipSuccess)
       return e;
     hipLaunchKernelGGL(k_norm_to_frag, dim3(npad), dim3(256), 0, s, b.x, m.ffn_norm[L], n, H,
-                       round_up(H, 256), m.eps, b.xb, b.part, pending);
+                       round_up(H, kq), quad, m.eps, b.xb, b.part, pending);
     pending = 0;
     // h = silu(gate . xn) * (up . xn) as the down GEMM's X: in the gate/up
     // GEMM's epilogue (into xh: other blocks are still reading xb), or,
-    // for batches on the ring kernel and mixed gate/up types, g and u
+    // for short batches and mixed gate/up types, g and u
     // then k_swiglu_to_frag
     const uint16_t *hx = b.xh;
     e = launch_gemm_bf16_swiglu(m.wgate[L], m.wup[L], b.xb, n, b.xh, num_cus, s);
@@ -671,9 +685,9 @@ hipError_t launch_prefill(const DecodeLaunch &m, const PrefillBufs &b, const int
       const gq_weight *gu[2] = {m.wgate[L], m.wup[L]};
       float *guo[2] = {b.g, b.u};
       if ((e = launch_gemm_bf16(gu, guo, 2, b.xb, n, b.part, false, num_cus, s)) != hipSuccess) return e;
-      const int kpf = round_up(F, 256);
+      const int kpf = round_up(F, kq);
       hipLaunchKernelGGL(k_swiglu_to_frag, dim3((int)(((long)npad / 16 * (kpf / 32) + 3) / 4)), dim3(256), 0,
-                         s, b.g, b.u, n, F, npad, kpf, b.xb);
+                         s, b.g, b.u, n, F, npad, kpf, quad, b.xb);
       hx = b.xb;
     } else if (e != hipSuccess) {
       return e;

@@ -82,6 +82,32 @@ def test_gemm_bf16(backend, orc, rows, k, n):
     check(Y, ref32, "bf16 vs fp32 CPU path", tol=1e-2)
 
 
+@pytest.mark.parametrize("dtype,rows,k,n", [
+    (Q4_K, 113, 5120, 1), (Q6_K, 97, 1280, 16), (13, 225, 2304, 17), (8, 111, 4128, 33), (Q4_K, 1, 256, 50),
+    (Q6_K, 500, 3072, 81), (13, 112, 1024, 96), (8, 130, 1056, 97), (Q4_K, 3001, 1792, 128), (Q6_K, 16, 9728, 128)])
+def test_gemm_bf16_short(backend, orc, dtype, rows, k, n):
+    """Batches of up to 128 tokens: every number of token tiles, row tiles of
+    112 with remainders, last quads of 1 to 4 units, K split or not."""
+    import gq
+    say(f"gemm bf16 short dtype={dtype} rows={rows} k={k} n={n}")
+    w, X, Wf, Y = run(backend, orc, rows, k, n, gq.GQ_GEMM_BF16, seed=rows + 3 * k + n, dtype=dtype)
+    ref = bf16_round(X).astype(np.float64) @ bf16_round(Wf).astype(np.float64).T
+    check(Y, ref, "bf16 vs same-operand fp64")
+
+
+def test_gemm_bf16_short_experts(backend, orc):
+    """Stacked experts of 24 rows (the wave-tiled layout) in a short batch."""
+    import gq
+    import torch
+    E, f, k, n = 3, 24, 512, 19
+    w = syn.make_blocks(Q4_K, E * f, k, seed=9)
+    X = syn.make_x(k, seed=10, batch=n)
+    h = backend.upload_experts(Q4_K, w, k, f, E)
+    Y = h.launch_only_batch(torch.from_numpy(X).cuda(), mode=gq.GQ_GEMM_BF16).cpu().numpy()
+    Wf = orc.dequant(Q4_K, w.reshape(-1), E * f * k).reshape(E * f, k)
+    check(Y, bf16_round(X).astype(np.float64) @ bf16_round(Wf).astype(np.float64).T, "experts vs same-operand fp64")
+
+
 @pytest.mark.parametrize("dtype,rows,k,n", [(Q4_K,) + sh for sh in SHAPES] + [(Q6_K,) + sh for sh in Q6_SHAPES]
                          + [(Q6_K, 3584, 18944, 512)])
 def test_gemm_int8(backend, orc, dtype, rows, k, n):
