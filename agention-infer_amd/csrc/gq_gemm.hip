@@ -12,20 +12,13 @@
 //                bf16 into LDS; X is converted to bf16 once (round to
 //                nearest even) by a prepass.  v_mfma_f32_16x16x32_bf16,
 //                fp32 accumulation.
-//  GQ_GEMM_INT8  X is packed per 32 elements exactly as KvDtype::Q8_0::pack
-//                (src/model/mod.rs:574-583): f16 scale xs, int8 q.  W
-//                nibbles (0..15) go to LDS as int8.  Each 32-element
-//                sub-block is one v_mfma_i32_16x16x32_i8 (exact integer
-//                dot); its result is scaled by (d*sc)*xs and the min term
-//                dmin*m*xs*sum(q) is subtracted in fp32.
+//  GQ_GEMM_INT8  gq_gemm_q8.hip.
 //
 // Tiling (bf16): a block computes 160 weight rows x 256 tokens (18944 rows
 // x 512 tokens -> 238 blocks, one round on 256 CUs).  K advances 64
 // elements (one Q4_K group) per stage, X fragments come straight from L2 into
 // the multiply waves' registers.  Batches of up to 128 tokens take
 // gq_gemm_quad.hip's kernel instead.
-// int8 (k_gemm_i8_direct): 160 rows x 256 tokens, W nibbles straight to
-// int8 MFMA, per-32 scaling on the VALU.
 #include <algorithm>
 #include <type_traits>
 
@@ -578,406 +571,6 @@ __global__ void k_gemm_reduce(ReduceSegs r, int ksplit, int add) {
   }
 }
 
-// ----------------------------------------------------------- int8 kernel
-// X fp32 [n][k] -> per-32 Q8 (KvDtype::Q8_0::pack: amax / 127, f16 scale,
-// codes from the f32 scale) in MFMA B-operand fragments for
-// v_mfma_i32_16x16x32_i8: fragment (token tile nt, 32-k block kb) is 64
-// lane slots of 8 codes (lane l: token 16 nt + l % 16, k 32 kb + 8 (l / 16)),
-// 512 B, ordered [nt][kb]; beside it, per (nt, kb), 16 records
-// (xs, xs * sum(q)) with xs the f16-rounded scale.  Tokens past n get
-// zero records.  One thread per 8 consecutive k of one token; the 4
-// threads of a 32-block are consecutive lanes.
-__global__ void k_x_to_q8_frag(const float *X, int n, int npad, int k, int kpad, int8_t *q,
-                               float2 *xr) {
-  const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  const int g8 = kpad / 8;
-  const bool ok = i < (long)npad * g8;
-  const int t = ok ? (int)(i / g8) : 0, c0 = ok ? (int)(i % g8) * 8 : 0;
-  float v[8];
-#pragma unroll
-  for (int e = 0; e < 8; e++) v[e] = ok && t < n && c0 + e < k ? X[(long)t * k + c0 + e] : 0.f;
-  float amax = 0.f;
-#pragma unroll
-  for (int e = 0; e < 8; e++) amax = fmaxf(amax, fabsf(v[e]));
-  amax = fmaxf(amax, __shfl_xor(amax, 1, 64));
-  amax = fmaxf(amax, __shfl_xor(amax, 2, 64));
-  const float s = amax > 0.f ? amax / 127.0f : 1.0f;
-  uint32_t w[2] = {0, 0};
-  int sum = 0;
-#pragma unroll
-  for (int e = 0; e < 8; e++) {
-    float r = roundf(v[e] / s);
-    r = fminf(fmaxf(r, -127.f), 127.f);
-    const int qi = (int)r;
-    sum += qi;
-    w[e >> 2] |= ((uint32_t)qi & 0xFFu) << (8 * (e & 3));
-  }
-  sum += __shfl_xor(sum, 1, 64);
-  sum += __shfl_xor(sum, 2, 64);
-  if (!ok) return;
-  const int nt = t >> 4, kb = c0 >> 5, sub = (c0 & 31) >> 3;
-  const long f = (long)nt * (kpad / 32) + kb;
-  *(uint2 *)(q + f * 512 + ((t & 15) + 16 * sub) * 8) = make_uint2(w[0], w[1]);
-  if (sub == 0) {
-    const float xs = t < n ? __half2float(__float2half_rn(s)) : 0.f;
-    xr[f * 16 + (t & 15)] = make_float2(xs, xs * (float)sum);
-  }
-}
-
-// Block tile 160 rows x 256 tokens, 512 threads = 8 waves, each both
-// multiplying and scaling: wave w owns rows 80 (w & 1) .. + 79 and tokens
-// 64 (w >> 1) .. + 63 (5 x 4 tiles of 16 x 16), so a SIMD's two waves
-// overlap one's scaling VALU with the other's MFMAs.  K-steps ("stages")
-// of 64 = one Q4_K group = two 32-element sub-blocks.  Per stage:
-//   * every thread fetches one 16-byte chunk of the block's W rows (the
-//     group's header or one of its two quant chunks, ggml order) a stage
-//     ahead and, after the stage's MFMAs, writes it to LDS: quant bytes as
-//     int8 A fragments (low nibbles = sub-block 0, high = sub-block 1; no
-//     scaling), the header as (d sc, dmin m) per row and sub-block;
-//   * each wave loads its X fragments and (xs, xs sum q) records from
-//     global memory (L2) straight into registers, a stage ahead;
-//   * per sub-block and tile, one v_mfma_i32_16x16x32_i8 gives the exact
-//     integer dot D, and y += (d sc) xs D in fp32 (VALU); the min term
-//     - (dmin m) xs sum(q) goes through an fp32 MFMA every two stages.
-// One barrier per stage.
-constexpr int I8M = 160, I8N = 256;
-__global__ __launch_bounds__(512) void k_gemm_i8_direct(const uint8_t *rec, int rows, int ntiles,
-                                                        const int8_t *xq, const float2 *xr, int n,
-                                                        int kpad, float *Y) {
-  __shared__ __align__(16) uint8_t Aq[2][2 * 10 * 512];      // [buf][ks][row tile] fragments
-  __shared__ __align__(16) float2 Ws[2][2][I8M];              // [buf][ks][row] (d sc, dmin m)
-  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int bid = xcd_block(blockIdx.x, gridDim.x), ntile = bid % ntiles, tile = bid / ntiles;
-  const int m0 = tile * I8M, n0 = ntile * I8N;
-  const int stages = kpad / 64, kb_all = kpad / 32;
-  const long row_stride = (long)(stages / 4) * 144;
-  // W chunk of this thread: row wr, chunk wc (0 header, 1-2 quants)
-  const bool wact = tid < 3 * I8M;
-  const int wr = wact ? tid / 3 : 0, wc = wact ? tid % 3 : 0;
-  const bool wok = wact && m0 + wr < rows;
-  const uint8_t *wsrc = rec + (long)min(m0 + wr, rows - 1) * row_stride;
-  auto load_w = [&](int s) -> uint4 {
-    const long off = (long)(s >> 2) * 144 + (wc == 0 ? 0 : 16 + 32 * (s & 3) + 16 * (wc - 1));
-    return *(const uint4 *)(wsrc + off);
-  };
-  auto store_w = [&](int s, int buf, uint4 c) {
-    if (!wact) return;
-    if (wc == 0) {
-      const int j = s & 3;
-      uint32_t sc0, mn0, sc1, mn1;
-      scale_min_k4(2 * j, c.y, c.z, c.w, sc0, mn0);
-      scale_min_k4(2 * j + 1, c.y, c.z, c.w, sc1, mn1);
-      const float d = h2f(c.x), dmin = h2f(c.x >> 16);
-      Ws[buf][0][wr] = wok ? make_float2(d * (float)sc0, dmin * (float)mn0) : make_float2(0.f, 0.f);
-      Ws[buf][1][wr] = wok ? make_float2(d * (float)sc1, dmin * (float)mn1) : make_float2(0.f, 0.f);
-    } else {
-      // bytes 16 (wc - 1) + b: element 16 (wc - 1) + b (low nibble, sub-block 0)
-      // and 32 + 16 (wc - 1) + b (high nibble, sub-block 1); k within the
-      // sub-block 16 (wc - 1) + b -> lane slot (row % 16) + 16 * (k / 8)
-      const uint32_t qw[4] = {c.x, c.y, c.z, c.w};
-      const int rt = wr >> 4, slot0 = (wr & 15) + 32 * (wc - 1);
-#pragma unroll
-      for (int h = 0; h < 2; h++) {
-        uint8_t *fr = &Aq[buf][(h * 10 + rt) * 512];
-        const uint32_t l0 = (qw[0] >> (4 * h)) & 0x0F0F0F0Fu, l1 = (qw[1] >> (4 * h)) & 0x0F0F0F0Fu;
-        const uint32_t l2 = (qw[2] >> (4 * h)) & 0x0F0F0F0Fu, l3 = (qw[3] >> (4 * h)) & 0x0F0F0F0Fu;
-        *(uint2 *)(fr + slot0 * 8) = make_uint2(l0, l1);
-        *(uint2 *)(fr + (slot0 + 16) * 8) = make_uint2(l2, l3);
-      }
-    }
-  };
-  // X: fragments (token tile 16-token nt, 32-k block kb) at xq + (nt * kb_all + kb) * 512
-  const int wm = wave & 1, wn = wave >> 1;
-  const long nt0 = (n0 >> 4) + 4 * wn;
-  struct XReg {
-    long b[2][4];
-    float2 r[2][4];
-  };
-  auto load_x = [&](int s, XReg &x) {
-#pragma unroll
-    for (int ks = 0; ks < 2; ks++)
-#pragma unroll
-      for (int jn = 0; jn < 4; jn++) {
-        const long f = (nt0 + jn) * kb_all + 2 * s + ks;
-        x.b[ks][jn] = *(const long *)(xq + f * 512 + lane * 8);
-        x.r[ks][jn] = xr[f * 16 + (lane & 15)];
-      }
-  };
-  f32x4_t acc[5][4];
-#pragma unroll
-  for (int i = 0; i < 5; i++)
-#pragma unroll
-    for (int jn = 0; jn < 4; jn++) acc[i][jn] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-  // Tiles t = 5 ks + i in a software pipeline: the MFMAs of tile t are
-  // issued before the scaling of tile t - 1, so the scaling VALU never
-  // waits for the integer results it needs.
-  auto compute = [&](int buf, const XReg &x) {
-    i32x4_t dq[2][4];
-    float ws[2][4];
-    auto mf = [&](int t) {
-      const int ks = t / 5, rt = 5 * wm + t % 5;
-      const long a = *(const long *)&Aq[buf][(ks * 10 + rt) * 512 + lane * 8];
-      const float4 w01 = *(const float4 *)&Ws[buf][ks][16 * rt + 4 * (lane >> 4)];
-      const float4 w23 = *(const float4 *)&Ws[buf][ks][16 * rt + 4 * (lane >> 4) + 2];
-      ws[t & 1][0] = w01.x;
-      ws[t & 1][1] = w01.z;
-      ws[t & 1][2] = w23.x;
-      ws[t & 1][3] = w23.z;
-#pragma unroll
-      for (int jn = 0; jn < 4; jn++) {
-        const i32x4_t z = {0, 0, 0, 0};
-        dq[t & 1][jn] = __builtin_amdgcn_mfma_i32_16x16x32_i8(a, x.b[ks][jn], z, 0, 0, 0);
-      }
-    };
-    auto scale = [&](int t) {
-      const int ks = t / 5, i = t % 5;
-#pragma unroll
-      for (int jn = 0; jn < 4; jn++) {
-        const float xs = x.r[ks][jn].x;
-#pragma unroll
-        for (int r = 0; r < 4; r++)
-          acc[i][jn][r] = fmaf(ws[t & 1][r] * xs, (float)dq[t & 1][jn][r], acc[i][jn][r]);
-        // keep the update here (not sunk below later tiles' MFMAs, which
-        // would keep every tile's integer result live at once)
-        asm volatile("" : "+v"(acc[i][jn]));
-      }
-    };
-    mf(0);
-    __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-    for (int t = 1; t < 10; t++) {
-      mf(t);
-      scale(t - 1);
-      __builtin_amdgcn_sched_barrier(0);
-    }
-    scale(9);
-  };
-  // prologue: stage 0 to LDS; each stage then loads its X and the next
-  // stage's W while it computes
-  {
-    const uint4 c = load_w(0);
-    store_w(0, 0, c);
-  }
-  __syncthreads();
-  // The min term -sum_sb (dmin m)[row][sb] (xs sum q)[token][sb] is a small
-  // product over the sub-blocks: every two stages (4 sub-blocks, both W
-  // slots of LDS still valid) one v_mfma_f32_16x16x4_f32 per tile adds it,
-  // lane l giving row l % 16 of -(dmin m) and token l % 16 of xs sum q for
-  // sub-block l / 16 (stages is a multiple of 4: kpad is whole units).
-  // The previous stage's LDS slot is being refilled with the next stage's W
-  // by other waves during an odd stage, so its (dmin m) values are taken
-  // into registers at the even stage.
-  const int sbl = lane >> 4;
-  float xmp[2][4];  // xs sum q of the previous stage, per (ks, token tile)
-  float amp[5];     // -(dmin m) of the previous stage, per row tile (lanes sbl < 2)
-  auto mins = [&](int kt, const XReg &x) {
-    const int mks = sbl & 1;
-    float bq[4];
-#pragma unroll
-    for (int jn = 0; jn < 4; jn++) {
-      const float p0 = mks ? xmp[1][jn] : xmp[0][jn];
-      const float c0 = mks ? x.r[1][jn].y : x.r[0][jn].y;
-      bq[jn] = sbl < 2 ? p0 : c0;
-    }
-#pragma unroll
-    for (int i = 0; i < 5; i++) {
-      const float am = sbl < 2 ? amp[i] : -Ws[kt & 1][mks][16 * (5 * wm + i) + (lane & 15)].y;
-#pragma unroll
-      for (int jn = 0; jn < 4; jn++)
-        acc[i][jn] = __builtin_amdgcn_mfma_f32_16x16x4f32(am, bq[jn], acc[i][jn], 0, 0, 0);
-    }
-  };
-  // X of stage kt + 1 is loaded while stage kt computes (two register sets,
-  // the loop unrolled by two).
-  auto stage = [&](int kt, const XReg &x, XReg &xn) {
-    uint4 c = make_uint4(0, 0, 0, 0);
-    if (kt + 1 < stages) {
-      c = load_w(kt + 1);
-      load_x(kt + 1, xn);
-    }
-    __builtin_amdgcn_sched_barrier(0);
-    compute(kt & 1, x);
-    if (kt & 1) {
-      mins(kt, x);
-    } else {
-#pragma unroll
-      for (int jn = 0; jn < 4; jn++) {
-        xmp[0][jn] = x.r[0][jn].y;
-        xmp[1][jn] = x.r[1][jn].y;
-      }
-#pragma unroll
-      for (int i = 0; i < 5; i++) amp[i] = -Ws[kt & 1][sbl & 1][16 * (5 * wm + i) + (lane & 15)].y;
-    }
-    if (kt + 1 < stages) store_w(kt + 1, (kt + 1) & 1, c);
-    __syncthreads();
-  };
-  XReg x0, x1;
-  load_x(0, x0);
-  for (int kt = 0; kt < stages; kt += 2) {  // stages is even (a multiple of 4)
-    stage(kt, x0, x1);
-    stage(kt + 1, x1, x0);
-  }
-  // D layout: lane holds rows 4 (lane / 16) + r of token column lane % 16.
-#pragma unroll
-  for (int i = 0; i < 5; i++) {
-    const int m = m0 + 80 * wm + 16 * i + 4 * (lane >> 4);
-#pragma unroll
-    for (int jn = 0; jn < 4; jn++) {
-      const int t = n0 + 64 * wn + 16 * jn + (lane & 15);
-      if (t >= n) continue;
-      float *yp = Y + (long)t * rows + m;
-      if (m + 3 < rows && (rows & 3) == 0) {
-        *(float4 *)yp = make_float4(acc[i][jn][0], acc[i][jn][1], acc[i][jn][2], acc[i][jn][3]);
-      } else {
-#pragma unroll
-        for (int r = 0; r < 4; r++)
-          if (m + r < rows) yp[r] = acc[i][jn][r];
-      }
-    }
-  }
-}
-
-// ----------------------------------------------------------- int8 kernel, Q6_K
-// Q6_K weights against the same per-32 Q8 activation fragments.  A Q6_K
-// code minus 32 is an int8 (-32..31), so the A operand is the codes
-// themselves.  Its scales change every 16 elements, half a 32-deep MFMA
-// step: each step runs twice with the other group's half of A zeroed
-// (lanes 0-31 hold k 0..15, lanes 32-63 k 16..31), and the two integer dots
-// are combined exactly, sc_a * D_a + sc_b * D_b (|D| <= 16 * 32 * 127),
-// before y += (d xs) * that in fp32.
-// Block tile 64 rows x 64 tokens, 256 threads; wave w owns rows 16 w ..
-// 16 w + 15 and all 64 tokens (4 MFMA tiles).  Per 64-element stage, a
-// stage ahead, every operand goes through LDS:
-//   * threads 0-127 (row tid / 2, half tid % 2) fetch the stage record's
-//     quant chunks of their row and write the half's 32 codes as int8 A
-//     fragments; threads 128-191 fetch the row's 4 group scales and d;
-//   * every thread fetches 16 bytes of the stage's X fragments (4 KiB) and
-//     threads 0-127 its 128 X scales.
-// One barrier per stage.
-constexpr int Q6M = 64, Q6N = 64, Q6J = Q6N / 16;
-__global__ __launch_bounds__(256) void k_gemm_i8_q6k(const uint8_t *rec, int rows, const int8_t *xq,
-                                                     const float2 *xr, int n, int kpad, float *Y) {
-  __shared__ __align__(16) uint8_t Aq[2][2][4][512];  // [buf][half][row tile][lane slot x 8 codes]
-  __shared__ __align__(16) int Sc[2][4][Q6M];         // [buf][group][row] int8 scale
-  __shared__ __align__(16) float Dd[2][Q6M];          // [buf][row] f16 d
-  __shared__ __align__(16) float Xs[2][2][Q6J][16];   // [buf][half][token tile][token] f16 xs
-  __shared__ __align__(16) uint8_t Xb[2][2][Q6J][512];  // [buf][half][token tile] B fragments
-  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int m0 = blockIdx.x * Q6M, n0 = blockIdx.y * Q6N;
-  const int stages = kpad / 64, kb_all = kpad / 32;
-  const long row_stride = (long)stages * 64;
-  // staging role of this thread
-  const int sr = tid < 128 ? tid >> 1 : tid - 128, sh = tid & 1;
-  const bool sq = tid < 128, ss = tid >= 128 && tid < 192;
-  const bool sok = m0 + sr < rows;
-  const uint8_t *srow = rec + (long)min(m0 + min(sr, Q6M - 1), rows - 1) * row_stride;
-  // the next stage's staged loads: the row's quant chunks (c1, c2, hb) or
-  // its scales and d (c0), one X scale (xsv), 16 bytes of X fragments (xf)
-  uint4 c1 = make_uint4(0, 0, 0, 0), c2 = c1, c0 = c1, xf = c1;
-  uint2 hb = make_uint2(0, 0);
-  float xsv = 0.f;
-  auto load_w = [&](int s) {
-    const uint8_t *rp = srow + (long)s * 64;
-    if (sq) {
-      c1 = *(const uint4 *)(rp + 16);
-      c2 = *(const uint4 *)(rp + 32);
-      hb = *(const uint2 *)(rp + 48 + 8 * sh);
-    } else if (ss) {
-      c0 = *(const uint4 *)rp;
-    }
-    if (tid < 32 * Q6J) {
-      const long f = ((n0 >> 4) + ((tid >> 4) % Q6J)) * kb_all + 2 * s + tid / (16 * Q6J);
-      xsv = xr[f * 16 + (tid & 15)].x;
-    }
-    if (tid < 64 * Q6J) {  // fragment (half, token tile) = tid / 32 (half-major), bytes 16 (tid % 32)
-      const int fi = tid >> 5, h = fi / Q6J, jn = fi % Q6J;
-      const long f = ((n0 >> 4) + jn) * kb_all + 2 * s + h;
-      xf = *(const uint4 *)(xq + f * 512 + 16 * (tid & 31));
-    }
-  };
-  auto store_w = [&](int buf) {
-    if (sq) {
-      // element e = 16 qq + i of half sh: low 4 bits = nibble sh of byte i
-      // of chunk 1 + qq, high 2 bits = bits 2i, 2i + 1 of dword 2 sh + qq
-      const uint32_t lw[2][4] = {{c1.x, c1.y, c1.z, c1.w}, {c2.x, c2.y, c2.z, c2.w}};
-      const uint32_t hw[2] = {hb.x, hb.y};
-      uint8_t *fr = &Aq[buf][sh][sr >> 4][0];
-#pragma unroll
-      for (int j = 0; j < 4; j++) {  // codes 8 j .. 8 j + 7: lane slot (row % 16) + 16 j
-        const int qq = j >> 1;
-        uint32_t out[2];
-#pragma unroll
-        for (int e = 0; e < 2; e++) {
-          const int i0 = 8 * (j & 1) + 4 * e;  // first of 4 elements within the 16
-          const uint32_t lo = (lw[qq][i0 >> 2] >> (4 * sh)) & 0x0F0F0F0Fu;
-          const uint32_t b2 = (hw[qq] >> (2 * i0)) & 0xFFu;
-          const uint32_t hi = (b2 | (b2 << 6) | (b2 << 12) | (b2 << 18)) & 0x03030303u;
-          const uint32_t q6 = lo | (hi << 4);
-          out[e] = sok ? (((q6 | 0x80808080u) - 0x20202020u) ^ 0x80808080u) : 0u;  // q - 32
-        }
-        *(uint2 *)(fr + ((sr & 15) + 16 * j) * 8) = make_uint2(out[0], out[1]);
-      }
-    } else if (ss) {
-#pragma unroll
-      for (int g = 0; g < 4; g++) Sc[buf][g][sr] = (int)(int8_t)((c0.x >> (8 * g)) & 0xFFu);
-      Dd[buf][sr] = sok ? h2f(c0.y) : 0.f;
-    }
-    if (tid < 32 * Q6J) Xs[buf][tid / (16 * Q6J)][(tid >> 4) % Q6J][tid & 15] = xsv;
-    if (tid < 64 * Q6J) {
-      const int fi = tid >> 5;
-      *(uint4 *)&Xb[buf][fi / Q6J][fi % Q6J][16 * (tid & 31)] = xf;
-    }
-  };
-  f32x4_t acc[Q6J];
-#pragma unroll
-  for (int jn = 0; jn < Q6J; jn++) acc[jn] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-  const int rr0 = 16 * wave + 4 * (lane >> 4);  // this lane's output rows rr0 .. rr0 + 3 (block-local)
-  auto compute = [&](int buf) {
-#pragma unroll
-    for (int h = 0; h < 2; h++) {
-      const long a = *(const long *)&Aq[buf][h][wave][lane * 8];
-      const long aa = lane < 32 ? a : 0, ab = lane < 32 ? 0 : a;  // groups 2h and 2h + 1
-      int sca[4], scb[4];
-      float dd[4];
-#pragma unroll
-      for (int r = 0; r < 4; r++) {
-        sca[r] = Sc[buf][2 * h][rr0 + r];
-        scb[r] = Sc[buf][2 * h + 1][rr0 + r];
-        dd[r] = Dd[buf][rr0 + r];
-      }
-#pragma unroll
-      for (int jn = 0; jn < Q6J; jn++) {
-        const long bx = *(const long *)&Xb[buf][h][jn][lane * 8];
-        const i32x4_t z = {0, 0, 0, 0};
-        const i32x4_t da = __builtin_amdgcn_mfma_i32_16x16x32_i8(aa, bx, z, 0, 0, 0);
-        const i32x4_t db = __builtin_amdgcn_mfma_i32_16x16x32_i8(ab, bx, z, 0, 0, 0);
-        const float xs = Xs[buf][h][jn][lane & 15];
-#pragma unroll
-        for (int r = 0; r < 4; r++)
-          acc[jn][r] = fmaf(dd[r] * xs, (float)(sca[r] * da[r] + scb[r] * db[r]), acc[jn][r]);
-      }
-    }
-  };
-  load_w(0);
-  store_w(0);
-  __syncthreads();
-  for (int s = 0; s < stages; s++) {
-    const bool more = s + 1 < stages;
-    if (more) load_w(s + 1);  // a stage ahead
-    compute(s & 1);
-    if (more) store_w((s & 1) ^ 1);
-    __syncthreads();
-  }
-#pragma unroll
-  for (int jn = 0; jn < Q6J; jn++) {
-    const int t = n0 + 16 * jn + (lane & 15);
-    if (t >= n) continue;
-#pragma unroll
-    for (int r = 0; r < 4; r++)
-      if (m0 + rr0 + r < rows) Y[(long)t * rows + m0 + rr0 + r] = acc[jn][r];
-  }
-}
-
 // ----------------------------------------------------------- host side
 size_t gemm_records_bytes(const Layout &L) {
   return (size_t)L.rows * L.units * gemm_unit_bytes(L.dtype);
@@ -1068,6 +661,19 @@ size_t gemm_x_elems(int units, int n, bool quad) {
   return (size_t)((n + GEMM_NPAD - 1) / GEMM_NPAD * GEMM_NPAD) * units * 256;
 }
 
+namespace {
+hipError_t launch_reduce(ReduceSegs &r, int ksplit, bool add, hipStream_t st) {
+  int blocks = 0;
+  for (int i = 0; i < r.nseg; i++) {
+    r.blk0[i] = blocks;
+    blocks += (int)((r.count[i] / 4 + 255) / 256 + 1);
+  }
+  r.blk0[r.nseg] = blocks;
+  hipLaunchKernelGGL(k_gemm_reduce, dim3((unsigned)blocks), dim3(256), 0, st, r, ksplit, add ? 1 : 0);
+  return hipGetLastError();
+}
+}  // namespace
+
 size_t gemm_part_floats(const gq_weight *const *ws, int count, int n, int num_cus, bool add) {
   const GemmPlan p = gemm_plan(ws, count, n, num_cus);
   if (p.ksplit == 1 && !add) return 0;
@@ -1077,7 +683,6 @@ size_t gemm_part_floats(const gq_weight *const *ws, int count, int n, int num_cu
 }
 
 size_t gemm_workspace_bytes(const gq_weight *w, int n, int mode, int num_cus) {
-  const size_t kpad = (size_t)w->L.units * 256;
   if (mode == GQ_GEMM_BF16) {
     if (w->L.dtype != T_Q4_K && w->L.dtype != T_Q6_K && w->L.dtype != T_Q5_K && w->L.dtype != T_Q8_0)
       return (size_t)-1;
@@ -1085,9 +690,7 @@ size_t gemm_workspace_bytes(const gq_weight *w, int n, int mode, int num_cus) {
     return ((xb + 255) & ~(size_t)255) + gemm_part_floats(&w, 1, n, num_cus, false) * 4 + 256;
   }
   if (w->L.dtype != T_Q4_K && w->L.dtype != T_Q6_K) return (size_t)-1;
-  // int8: fragments [npad/16][kpad/32][512 B] + records [npad/16][kpad/32][16] float2
-  const size_t npad = (size_t)(n + I8N - 1) / I8N * I8N;
-  return ((npad * kpad + 255) & ~(size_t)255) + npad * (kpad / 32) * 8 + 256;
+  return gemm_q8_workspace_bytes(w->L, n, num_cus);
 }
 
 hipError_t launch_x_to_frag(const float *X, int n, int k, uint16_t *xb, hipStream_t st) {
@@ -1151,17 +754,21 @@ hipError_t launch_gemm_bf16(const gq_weight *const *ws, float *const *ys, int co
   }
   ReduceSegs r{};
   r.nseg = count;
-  int blocks = 0;
   for (int i = 0; i < count; i++) {
     r.part[i] = a.seg[i].part;
     r.y[i] = a.seg[i].y;
     r.count[i] = (long)n * a.seg[i].rows;
-    r.blk0[i] = blocks;
-    blocks += (int)((r.count[i] / 4 + 255) / 256 + 1);
   }
-  r.blk0[count] = blocks;
-  hipLaunchKernelGGL(k_gemm_reduce, dim3((unsigned)blocks), dim3(256), 0, st, r, p.ksplit, add ? 1 : 0);
-  return hipGetLastError();
+  return launch_reduce(r, p.ksplit, add, st);
+}
+
+hipError_t launch_gemm_reduce(const float *part, float *y, long count, int ksplit, hipStream_t st) {
+  ReduceSegs r{};
+  r.nseg = 1;
+  r.part[0] = part;
+  r.y[0] = y;
+  r.count[0] = count;
+  return launch_reduce(r, ksplit, false, st);
 }
 
 hipError_t launch_gemm_bf16_swiglu(const gq_weight *gate, const gq_weight *up, const uint16_t *xb, int n,
@@ -1205,7 +812,6 @@ hipError_t launch_gemm(const gq_weight *w, const float *X, int n, float *Y, int 
                        void *workspace, size_t ws_bytes, int num_cus, hipStream_t st) {
   (void)ws_bytes;
   const Layout &L = w->L;
-  const int kpad = L.units * 256;
   if (mode == GQ_GEMM_BF16) {
     uint16_t *xb = (uint16_t *)workspace;
     const bool quad = gemm_uses_quad(&w, 1, n);
@@ -1214,26 +820,8 @@ hipError_t launch_gemm(const gq_weight *w, const float *X, int n, float *Y, int 
     hipError_t e = quad ? launch_x_to_quad(X, n, L.k, xb, st) : launch_x_to_frag(X, n, L.k, xb, st);
     if (e != hipSuccess) return e;
     return launch_gemm_bf16(&w, &Y, 1, xb, n, part, false, num_cus, st);
-  } else {
-    if (!w->gemm_raw) return hipErrorInvalidValue;
-    const int npad = (n + I8N - 1) / I8N * I8N;
-    int8_t *xq = (int8_t *)workspace;
-    float2 *xr = (float2 *)((char *)workspace + (((size_t)npad * kpad + 255) & ~(size_t)255));
-    const long threads = (long)npad * (kpad / 8);
-    hipLaunchKernelGGL(k_x_to_q8_frag, dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, st, X,
-                       n, npad, L.k, kpad, xq, xr);
-    if (L.dtype == T_Q6_K) {
-      hipLaunchKernelGGL(k_gemm_i8_q6k, dim3((unsigned)((L.rows + Q6M - 1) / Q6M), (unsigned)((n + Q6N - 1) / Q6N)),
-                         dim3(256), 0, st, (const uint8_t *)w->gemm_raw, L.rows, (const int8_t *)xq,
-                         (const float2 *)xr, n, kpad, Y);
-      return hipGetLastError();
-    }
-    const int ntiles = npad / I8N, mtiles = (L.rows + I8M - 1) / I8M;
-    hipLaunchKernelGGL(k_gemm_i8_direct, dim3((unsigned)(mtiles * ntiles)), dim3(512), 0, st,
-                       (const uint8_t *)w->gemm_raw, L.rows, ntiles, (const int8_t *)xq,
-                       (const float2 *)xr, n, kpad, Y);
   }
-  return hipGetLastError();
+  return launch_gemm_q8(w, X, n, Y, workspace, num_cus, st);
 }
 
 }  // namespace gq

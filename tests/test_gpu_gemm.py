@@ -130,6 +130,33 @@ def test_gemm_int8(backend, orc, dtype, rows, k, n):
     check(Y[sub], ref32, "int8 vs fp32 CPU path", tol=3e-2)
 
 
+@pytest.mark.parametrize("dtype", [Q4_K, Q6_K])
+@pytest.mark.parametrize("rows,k,n", [(1, 256, 1), (161, 1536, 129), (321, 2560, 257), (2400, 768, 384), (159, 5000, 128)])
+def test_gemm_int8_tiles(backend, orc, dtype, rows, k, n):
+    """Both token tiles (128 and 256), one row past a tile and one short of
+    it, K splits of uneven units, a ragged last unit; Q6_K scales at both
+    ends of int8, where sc (q - 32) passes 11 bits, and activations whose
+    blocks differ by 2^30 in one unit."""
+    import gq
+    import torch
+    say(f"gemm int8 tiles dtype={dtype} rows={rows} k={k} n={n}")
+    rng = np.random.default_rng(rows + k + n)
+    w = syn.make_blocks(dtype, rows, k, seed=rows + n)
+    if dtype == Q6_K:
+        b = w.reshape(rows, -1, 210)
+        b[..., 192:208] = rng.integers(-128, 128, b[..., 192:208].shape, dtype=np.int8).view(np.uint8)
+    X = syn.make_x(k, seed=n, batch=n)
+    X[:, :32] *= np.float32(2.0 ** -30)
+    h = backend.upload_weight(dtype, w, k, rows)
+    Y = h.launch_only_batch(torch.from_numpy(X).cuda(), mode=gq.GQ_GEMM_INT8).cpu().numpy()
+    Wf = orc.dequant_rows(dtype, w, k).astype(np.float64)
+    Xq = np.zeros((n, (k + 31) // 32 * 32), np.float64)
+    for t in range(n):
+        sc, q = orc.quantize_q8_32(X[t])
+        Xq[t, :q.size] = q.astype(np.float64) * np.repeat(sc.view(np.float16).astype(np.float64), 32)[:q.size]
+    check(Y, Xq[:, :k] @ Wf.T, "int8 vs same-operand fp64")
+
+
 def test_gemm_full_config(backend, orc):
     """config 2: Q4_K 18944 x 3584 times 512 tokens, both modes."""
     import gq
