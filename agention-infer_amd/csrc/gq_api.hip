@@ -676,7 +676,7 @@ int gq_gemm(const gq_weight *w, const float *X_dev, int n, float *Y_dev, int mod
   if (n < 0) return fail(GQ_EINVAL, "negative batch");
   if (n == 0 || w->L.rows == 0) return GQ_OK;
   if (mode != GQ_GEMM_BF16 && mode != GQ_GEMM_INT8) return fail(GQ_EINVAL, "bad gemm mode %d", mode);
-  const size_t ws = gq::gemm_workspace_bytes(w, n, mode, g_dev.num_cus);
+  size_t ws = gq::gemm_workspace_bytes(w, n, mode, g_dev.num_cus);
   if (ws == (size_t)-1)
     return fail(GQ_EDTYPE, "gq_gemm: %s weights not supported in %s mode", type_name(w->L.dtype),
                 mode == GQ_GEMM_BF16 ? "bf16" : "int8");
@@ -684,6 +684,9 @@ int gq_gemm(const gq_weight *w, const float *X_dev, int n, float *Y_dev, int mod
     int rc2 = gq_ensure_gemm_records(w, (hipStream_t)stream);  // both modes read the ggml-order copy
     if (rc2) return rc2;
   }
+  // An eager call takes room for every call of up to n tokens, so that these
+  // may be captured afterwards.
+  if (!stream_capturing((hipStream_t)stream)) ws = std::max(ws, gq::gemm_workspace_bound(w, n, g_dev.num_cus));
   void *wsp = nullptr;
   if (ws && (rc = stream_workspace((hipStream_t)stream, ws, &wsp))) return rc;
   hipError_t e = gq::launch_gemm(w, X_dev, n, Y_dev, mode, wsp, ws, g_dev.num_cus,

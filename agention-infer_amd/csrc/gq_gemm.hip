@@ -693,6 +693,18 @@ size_t gemm_workspace_bytes(const gq_weight *w, int n, int mode, int num_cus) {
   return gemm_q8_workspace_bytes(w->L, n, num_cus);
 }
 
+// Bytes that serve any call on w of up to n tokens, in either mode.  (A
+// shorter batch has fewer blocks and so may split K further, into more
+// partial products than a longer one.)
+size_t gemm_workspace_bound(const gq_weight *w, int n, int num_cus) {
+  size_t b = gemm_workspace_bytes(w, n, GQ_GEMM_BF16, num_cus);
+  if (n > GEMM_QUAD_MAX) b = std::max(b, gemm_workspace_bytes(w, GEMM_QUAD_MAX, GQ_GEMM_BF16, num_cus));
+  for (int m = GEMM_NPAD; m < n; m += GEMM_NPAD)
+    b = std::max(b, gemm_workspace_bytes(w, m, GQ_GEMM_BF16, num_cus));
+  if (w->L.dtype == T_Q4_K || w->L.dtype == T_Q6_K) b = std::max(b, gemm_q8_workspace_bound(w->L, n, num_cus));
+  return b;
+}
+
 hipError_t launch_x_to_frag(const float *X, int n, int k, uint16_t *xb, hipStream_t st) {
   const int kpad = (k + 255) / 256 * 256;
   const int npad = (n + GEMM_NPAD - 1) / GEMM_NPAD * GEMM_NPAD;

@@ -404,28 +404,32 @@ struct Q8Plan {
 // x 3584 Q4_K at 512 tokens 197 / 142, at 128 62 / 74; 3584 x 18944 Q6_K at
 // 200 139 / 99; 9000 x 512 Q6_K at 300 26 / 31; 3584 x 3584 Q4_K at 512 61 / 48
 // (in 2 / 5 splits).
-Q8Plan q8_plan(const Layout &L, int n, int num_cus) {
-  Q8Plan p{};
-  p.tiles = (L.rows + Q8_ROWS - 1) / Q8_ROWS;
+double q8_split(const Layout &L, int nj, int n, int num_cus, int &ksplit) {
   const double out = (double)n * L.rows * 8e-6 / 4.5;  // one partial product written and read
+  const int bn = 128 * nj;
+  const long tiles = (long)((L.rows + Q8_ROWS - 1) / Q8_ROWS) * ((n + bn - 1) / bn);
   double best = 1e30;
-  for (int nj = 1; nj <= 2; nj++) {
-    const int bn = 128 * nj, nt = (n + bn - 1) / bn;
-    const long tiles = (long)p.tiles * nt;
-    for (int ks = 1; ks <= std::min(L.units, 16); ks++) {
-      const long rounds = (tiles * ks + num_cus - 1) / num_cus;
-      const double t =
-          rounds * (3.0 + (nj == 1 ? 6.5 : 10.0) * ((L.units + ks - 1) / ks)) + (ks > 1 ? 4.0 + ks * out : 0.0);
-      if (t < best - 1e-9) {
-        best = t;
-        p.nj = nj;
-        p.bn = bn;
-        p.ntiles = nt;
-        p.npad = nt * bn;
-        p.ksplit = ks;
-      }
+  for (int ks = 1; ks <= std::min(L.units, 16); ks++) {
+    const long rounds = (tiles * ks + num_cus - 1) / num_cus;
+    const double t =
+        rounds * (3.0 + (nj == 1 ? 6.5 : 10.0) * ((L.units + ks - 1) / ks)) + (ks > 1 ? 4.0 + ks * out : 0.0);
+    if (t < best - 1e-9) {
+      best = t;
+      ksplit = ks;
     }
   }
+  return best;
+}
+Q8Plan q8_plan(const Layout &L, int n, int num_cus) {
+  int k1 = 1, k2 = 1;
+  const double t1 = q8_split(L, 1, n, num_cus, k1), t2 = q8_split(L, 2, n, num_cus, k2);
+  Q8Plan p{};
+  p.nj = t2 < t1 - 1e-9 ? 2 : 1;
+  p.bn = 128 * p.nj;
+  p.ntiles = (n + p.bn - 1) / p.bn;
+  p.npad = p.ntiles * p.bn;
+  p.tiles = (L.rows + Q8_ROWS - 1) / Q8_ROWS;
+  p.ksplit = p.nj == 2 ? k2 : k1;
   return p;
 }
 template <int FMT>
@@ -449,6 +453,26 @@ Q8Bytes q8_bytes(const Q8Plan &p, const Layout &L, int n) {
 size_t gemm_q8_workspace_bytes(const Layout &L, int n, int num_cus) {
   const Q8Bytes b = q8_bytes(q8_plan(L, n, num_cus), L, n);
   return b.xq + b.xs + b.xm + b.part + 256;
+}
+
+// A bound for every batch of up to n tokens.  A token tile's batches share
+// their block counts, so the shortest has the largest split of each tile size.
+size_t gemm_q8_workspace_bound(const Layout &L, int n, int num_cus) {
+  Q8Plan p{};
+  p.npad = (n + 255) / 256 * 256;
+  p.ksplit = 1;
+  const Q8Bytes b = q8_bytes(p, L, n);
+  size_t part = 0;
+  for (int n0 = 0; n0 < n; n0 += 128) {
+    int ks = 1;
+    for (int nj = 1; nj <= 2; nj++) {
+      int k = 1;
+      (void)q8_split(L, nj, n0 + 1, num_cus, k);
+      ks = std::max(ks, k);
+    }
+    if (ks > 1) part = std::max(part, (size_t)ks * std::min(n, n0 + 128) * L.rows * 4);
+  }
+  return b.xq + b.xs + b.xm + part + 256;
 }
 
 hipError_t launch_gemm_q8(const gq_weight *w, const float *X, int n, float *Y, void *workspace, int num_cus,

@@ -214,8 +214,10 @@ hipError_t launch_quantize_row_q8k(const float *x, long n, float *d, int8_t *qs,
 hipError_t launch_gemm(const gq_weight *w, const float *X, int n, float *Y, int mode,
                        void *workspace, size_t ws_bytes, int num_cus, hipStream_t st);
 size_t gemm_workspace_bytes(const gq_weight *w, int n, int mode, int num_cus);
+size_t gemm_workspace_bound(const gq_weight *w, int n, int num_cus);  // any mode, up to n tokens
 // Its int8 mode (Q4_K, Q6_K).
 size_t gemm_q8_workspace_bytes(const Layout &L, int n, int num_cus);
+size_t gemm_q8_workspace_bound(const Layout &L, int n, int num_cus);
 hipError_t launch_gemm_q8(const gq_weight *w, const float *X, int n, float *Y, void *workspace, int num_cus,
                           hipStream_t st);
 // y[i] = sum_s part[s][i], s in order, i < count.

@@ -237,6 +237,35 @@ def test_gemm_errors_and_edges(backend):
         assert torch.all(y == 0)
 
 
+
+@pytest.mark.parametrize("mode", [0, 1])
+def test_gemm_capture_of_shorter_batches(backend, mode):
+    """One eager call of the largest batch, in either mode, leaves room for
+    capturing any shorter one, also where that splits K further."""
+    import torch
+    t, rows, k = Q4_K, 18944, 1024
+    h = backend.upload_weight(t, syn.make_blocks(t, rows, k, seed=71), k, rows)
+    X = torch.from_numpy(syn.make_x(k, seed=72, batch=512)).cuda()
+    Y = torch.zeros((512, rows), device="cuda")
+    s = torch.cuda.Stream()
+    torch.cuda.synchronize()
+    h.launch_only_batch(X, mode=1 - mode, Y_dev=Y, stream=s.cuda_stream)
+    s.synchronize()
+    for n in (129, 128, 40):
+        g = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(g, stream=s):
+            h.launch_only_batch(X[:n], mode=mode, Y_dev=Y[:n], stream=s.cuda_stream)
+        ref = torch.zeros((n, rows), device="cuda")
+        h.launch_only_batch(X[:n], mode=mode, Y_dev=ref, stream=s.cuda_stream)
+        s.synchronize()
+        for i in range(2):
+            Y.zero_()
+            torch.cuda.synchronize()
+            g.replay()
+            torch.cuda.synchronize()
+            assert torch.equal(Y[:n], ref), f"n {n} replay {i}"
+
+
 def test_gemm_capture_survives_workspace_growth(backend):
     """A HIP graph captured around gq_gemm keeps its workspace: a later,
     larger call on the same stream grows the stream's workspace without
