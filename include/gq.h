@@ -36,8 +36,8 @@ extern "C" {
 #define GQ_TYPE_IQ3_XXS 18
 
 /* gq_gemm modes (batched prefill). */
-#define GQ_GEMM_BF16 0  /* weight tiles dequantized to bf16 in LDS, bf16 MFMA */
-#define GQ_GEMM_INT8 1  /* activations packed per-32 to Q8, int8 MFMA      */
+#define GQ_GEMM_BF16 0  /* weights dequantized to bf16, bf16 MFMA            */
+#define GQ_GEMM_INT8 1  /* activations packed per-32 to Q8, exact products */
 
 typedef struct gq_weight gq_weight;
 
@@ -114,12 +114,14 @@ int gq_dequant_rows_host(const gq_weight *w, int row0, int nrows, float *out_hos
  * prefill path of WeightMap::matmul_batch_into (src/model/mod.rs:414-464):
  * X_dev [n][in_dim] fp32 token-major -> Y_dev [n][out_dim] fp32.
  * mode GQ_GEMM_BF16 (Q4_K, Q5_K, Q6_K or Q8_0 weights; each dequantized as
- * dequant_row does, then rounded to bf16) or GQ_GEMM_INT8 (Q4_K weights).
+ * dequant_row does, then rounded to bf16) or GQ_GEMM_INT8 (Q4_K or Q6_K).
  * The first call on a weight builds its GEMM copy (per-stage records) and
  * synchronizes the stream once.  The packed-X workspace is the stream's own
  * (as gq_moe_ffn's).  Under HIP graph capture a call is accepted only if
  * that first call was made before and the stream's workspace already holds
  * the call's bytes; otherwise it fails with GQ_EINVAL and records nothing.
+ * (An eager call takes room for every call on its weight of up to n tokens,
+ * in either mode.)
  * Workspaces are never freed while the process runs, so a captured graph
  * stays valid when later, larger calls grow the stream's workspace. */
 int gq_gemm(const gq_weight *w, const float *X_dev, int n, float *Y_dev, int mode, void *stream);
