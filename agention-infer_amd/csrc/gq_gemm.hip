@@ -701,7 +701,8 @@ size_t gemm_workspace_bound(const gq_weight *w, int n, int num_cus) {
   if (n > GEMM_QUAD_MAX) b = std::max(b, gemm_workspace_bytes(w, GEMM_QUAD_MAX, GQ_GEMM_BF16, num_cus));
   for (int m = GEMM_NPAD; m < n; m += GEMM_NPAD)
     b = std::max(b, gemm_workspace_bytes(w, m, GQ_GEMM_BF16, num_cus));
-  if (w->L.dtype == T_Q4_K || w->L.dtype == T_Q6_K) b = std::max(b, gemm_q8_workspace_bound(w->L, n, num_cus));
+  if (w->L.dtype == T_Q4_K || w->L.dtype == T_Q6_K) 
+    b = std::max(b, q8_bytes_bound(w->L.rows, w->L.units, n, num_cus));
   return b;
 }
 

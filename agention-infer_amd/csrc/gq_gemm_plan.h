@@ -1,0 +1,113 @@
+// gq_gemm_plan.h -- which kernel a batched product takes, how it is cut into
+// blocks, and the workspace it needs.  Host code without HIP, so that the
+// rules are tested against measured times on the CPU.
+#pragma once
+#include <stddef.h>
+
+#include <algorithm>
+
+namespace gq {
+
+// ----------------------------------------------------------- int8 mode
+// (gq_gemm_q8.hip.)  small: 64 x 64 blocks, no K split; else 160 rows x 128 nj
+// tokens.
+constexpr int Q8_ROWS = 160, Q6S = 64;
+struct Q8Plan {
+  bool small;
+  int nj, npad, ntiles, tiles, ksplit;
+};
+
+// The K split with the least estimated time of a token tile, us: rounds of
+// blocks, each a start and its units (6.5 or 10 us each), and the reduction's
+// launch and traffic.  Measured with 128- / 256-token tiles, us a call: 18944
+// x 3584 Q4_K at 512 tokens 197 / 142, at 128 62 / 74; 3584 x 18944 Q6_K at
+// 200 139 / 99; 9000 x 512 Q6_K at 300 26 / 31; 3584 x 3584 Q4_K at 512 61 / 48
+// (in 2 / 5 splits).
+inline double q8_split(int rows, int units, int nj, int n, int num_cus, int &ksplit) {
+  const double out = (double)n * rows * 8e-6 / 4.5;  // one partial product written and read
+  const int bn = 128 * nj;
+  const long tiles = (long)((rows + Q8_ROWS - 1) / Q8_ROWS) * ((n + bn - 1) / bn);
+  double best = 1e30;
+  for (int ks = 1; ks <= std::min(units, 16); ks++) {
+    const long rounds = (tiles * ks + num_cus - 1) / num_cus;
+    const double t =
+        rounds * (3.0 + (nj == 1 ? 6.5 : 10.0) * ((units + ks - 1) / ks)) + (ks > 1 ? 4.0 + ks * out : 0.0);
+    if (t < best - 1e-9) {
+      best = t;
+      ksplit = ks;
+    }
+  }
+  return best;
+}
+
+// Whether a Q6_K product takes the small kernel: where its estimated time is
+// less by more than the estimates' error (about 4%), us a call.  Its
+// blocks wait on latency, 4 us a unit, until they are more than the CUs; the
+// other kernel pays a longer start, its 160-row stages and (in p's split) a
+// reduction.  Measured small / 160-row, at 256 CUs: 600 x 256 at 200 tokens 11 /
+// 19, 4800 x 512 at 200 18 / 26, 2400 x 768 at 700 26 / 35, 9000 x 256 at 512
+// 26 / 22, 1200 x 1024 at 1024 31 / 28, 600 x 1024 at 8 22 / 17.
+inline bool q6_small(int rows, int units, int n, const Q8Plan &p, int num_cus) {
+  const double out = (double)n * rows * 8e-6 / 4.5;
+  const long blocks = (long)((rows + Q6S - 1) / Q6S) * ((n + Q6S - 1) / Q6S);
+  if ((n + Q6S - 1) / Q6S > 65535) return false;  // (the launch's second dimension)
+  const double small =
+      5.7 + units * (4.0 + (blocks > num_cus ? 0.65 + 1.46 * (blocks - num_cus) / num_cus : 0.0)) +
+      std::min(n, Q6S) / (double)Q6S + 0.95 * out;
+  const int bn = 128 * p.nj;
+  const long tiles = (long)((rows + Q8_ROWS - 1) / Q8_ROWS) * ((n + bn - 1) / bn) * p.ksplit;
+  const double rounds = (double)((tiles + num_cus - 1) / num_cus), upb = (units + p.ksplit - 1) / p.ksplit;
+  const double used = std::min(n, 128) / 128.0 * std::min(rows, Q8_ROWS) / Q8_ROWS;
+  const double big = 6.7 + 0.85 * tiles / (rounds * num_cus) +
+                     rounds * (3.85 + upb * ((p.nj == 1 ? 5.3 : 7.0) + 2.6 * used)) +
+                     (p.ksplit > 1 ? 1.2 + 1.06 * p.ksplit * out : 0.0) + 0.3 * out;
+  return small < 0.97 * big;
+}
+
+inline Q8Plan q8_plan(int dtype, int rows, int units, int n, int num_cus) {
+  int k1 = 1, k2 = 1;
+  const double t1 = q8_split(rows, units, 1, n, num_cus, k1), t2 = q8_split(rows, units, 2, n, num_cus, k2);
+  Q8Plan p{};
+  p.nj = t2 < t1 - 1e-9 ? 2 : 1;
+  p.ksplit = p.nj == 2 ? k2 : k1;
+  p.small = dtype == 14 && q6_small(rows, units, n, p, num_cus);
+  if (p.small) p.ksplit = 1;
+  const int bm = p.small ? Q6S : Q8_ROWS, bn = p.small ? Q6S : 128 * p.nj;
+  p.ntiles = (n + bn - 1) / bn;
+  p.npad = p.ntiles * bn;
+  p.tiles = (rows + bm - 1) / bm;
+  return p;
+}
+
+// Workspace: codes, scales, thirds, partial products.
+struct Q8Bytes {
+  size_t xq, xs, xm, part;
+  size_t total() const { return xq + xs + xm + part + 256; }
+};
+inline Q8Bytes q8_bytes(const Q8Plan &p, int rows, int units, int n) {
+  const auto up256 = [](size_t v) { return (v + 255) & ~(size_t)255; };
+  const size_t tu = (size_t)(p.npad / 16) * units;
+  return {up256(tu * (p.small ? 4096 : 8192)), up256(tu * 512), up256(tu * 1024),
+          p.ksplit > 1 ? (size_t)p.ksplit * n * rows * 4 : 0};
+}
+
+// A bound for every batch of up to n tokens.  A token tile's batches share
+// their block counts, so the shortest has the largest split of each tile size.
+inline size_t q8_bytes_bound(int rows, int units, int n, int num_cus) {
+  Q8Plan p{};
+  p.npad = (n + 255) / 256 * 256;
+  p.ksplit = 1;
+  Q8Bytes b = q8_bytes(p, rows, units, n);
+  for (int n0 = 0; n0 < n; n0 += 128) {
+    int ks = 1;
+    for (int nj = 1; nj <= 2; nj++) {
+      int k = 1;
+      (void)q8_split(rows, units, nj, n0 + 1, num_cus, k);
+      ks = std::max(ks, k);
+    }
+    if (ks > 1) b.part = std::max(b.part, (size_t)ks * std::min(n, n0 + 128) * rows * 4);
+  }
+  return b.total();
+}
+
+}  // namespace gq

@@ -49,7 +49,9 @@ namespace {
 // [npad/16][kpad/32][16]; and (Q4_K) xs sum(q) in bf16 thirds
 // [npad/16][kpad/256][64][8] (lane l: token l % 16, third l / 16, the unit's 8
 // blocks; zeros for l >= 48).  Tokens past n are all zero.  A wave packs one
-// fragment.
+// fragment.  I8 (the small kernel): the codes as int8 in the elements' order,
+// [npad/16][kpad/32][64][8 bytes].
+template <bool I8>
 __global__ __launch_bounds__(256) void k_x_to_q8(const float *X, int n, int npad, int k, int units, uint16_t *xq,
                                                  float *xs, uint16_t *xm) {
   const int lane = threadIdx.x & 63, kbs = 8 * units;
@@ -76,21 +78,26 @@ __global__ __launch_bounds__(256) void k_x_to_q8(const float *X, int n, int npad
   amax = fmaxf(amax, __shfl_xor(amax, 16, 64));
   amax = fmaxf(amax, __shfl_xor(amax, 32, 64));
   const float s = amax > 0.f ? amax / 127.0f : 1.0f;
-  float q[8];
-  int sum = 0;
+  int q[8], sum = 0;
 #pragma unroll
   for (int e = 0; e < 8; e++) {
-    const int c = (int)fminf(fmaxf(roundf(v[e] / s), -127.f), 127.f);
-    sum += c;
-    q[e] = (float)c;
+    q[e] = (int)fminf(fmaxf(roundf(v[e] / s), -127.f), 127.f);
+    sum += q[e];
+  }
+  const float sc = t < n ? __half2float(__float2half_rn(s)) : 0.f;
+  if (sub == 0) xs[f * 16 + lane] = sc;
+  if constexpr (I8) {
+    uint32_t w[2] = {0, 0};
+#pragma unroll
+    for (int e = 0; e < 8; e++) w[e >> 2] |= ((uint32_t)q[e] & 0xFFu) << (8 * (e & 3));
+    *(uint2 *)((uint8_t *)xq + (f * 64 + lane) * 8) = make_uint2(w[0], w[1]);
+    return;
   }
   sum += __shfl_xor(sum, 16, 64);
   sum += __shfl_xor(sum, 32, 64);
-  h16x8_t o = {(_Float16)q[0], (_Float16)q[2], (_Float16)q[1], (_Float16)q[3],
-               (_Float16)q[4], (_Float16)q[6], (_Float16)q[5], (_Float16)q[7]};
+  h16x8_t o = {(_Float16)(float)q[0], (_Float16)(float)q[2], (_Float16)(float)q[1], (_Float16)(float)q[3],
+               (_Float16)(float)q[4], (_Float16)(float)q[6], (_Float16)(float)q[5], (_Float16)(float)q[7]};
   *(h16x8_t *)(xq + (f * 64 + lane) * 8) = o;
-  const float sc = t < n ? __half2float(__float2half_rn(s)) : 0.f;
-  if (sub == 0) xs[f * 16 + lane] = sc;
   if (xm) {
     const float x = sc * (float)sum, x1 = __uint_as_float(f2bf(x) << 16), x2 = __uint_as_float(f2bf(x - x1) << 16);
     xm[(((long)nt * units + (kb >> 3)) * 64 + lane) * 8 + (kb & 7)] =
@@ -104,10 +111,9 @@ struct Q8Args {
   const uint16_t *xq, *xm;
   const float *xs;
   float *y, *part;        // part: partial products [ksplit][n][rows] instead
-  int rows, n, kpad, ntiles, tiles, ksplit;
+  int rows, n, kpad, ntiles, ksplit;
 };
 
-constexpr int Q8_ROWS = 160;  // rows per block; 128 NJ tokens
 
 __device__ __forceinline__ uint32_t pkfma(uint32_t a, h16x2_t s, h16x2_t c) {
   const h16x2_t v = __builtin_bit_cast(h16x2_t, a);
@@ -394,93 +400,155 @@ __global__ __launch_bounds__(512) void k_gemm_q8(Q8Args a) {
   }
 }
 
-// 128 or 256 tokens per block, and the rest of a launch's shape.
-struct Q8Plan {
-  int nj, bn, npad, ntiles, tiles, ksplit;
-};
-// The token tile and K split with the least estimated time, us: rounds of
-// blocks, each a start and its units (6.5 or 10 us each), and the reduction's
-// launch and traffic.  Measured with 128- / 256-token tiles, us a call: 18944
-// x 3584 Q4_K at 512 tokens 197 / 142, at 128 62 / 74; 3584 x 18944 Q6_K at
-// 200 139 / 99; 9000 x 512 Q6_K at 300 26 / 31; 3584 x 3584 Q4_K at 512 61 / 48
-// (in 2 / 5 splits).
-double q8_split(const Layout &L, int nj, int n, int num_cus, int &ksplit) {
-  const double out = (double)n * L.rows * 8e-6 / 4.5;  // one partial product written and read
-  const int bn = 128 * nj;
-  const long tiles = (long)((L.rows + Q8_ROWS - 1) / Q8_ROWS) * ((n + bn - 1) / bn);
-  double best = 1e30;
-  for (int ks = 1; ks <= std::min(L.units, 16); ks++) {
-    const long rounds = (tiles * ks + num_cus - 1) / num_cus;
-    const double t =
-        rounds * (3.0 + (nj == 1 ? 6.5 : 10.0) * ((L.units + ks - 1) / ks)) + (ks > 1 ? 4.0 + ks * out : 0.0);
-    if (t < best - 1e-9) {
-      best = t;
-      ksplit = ks;
+// ----------------------------------------------------------- small kernel
+// Q6_K launches that leave the kernel above mostly idle: a short depth, or few
+// rows and tokens.  There the latency of a stage counts and not the rate, and
+// a 160-row stage is a long one; a block here is 64 rows x 64 tokens on int8
+// MFMA, 4 waves, each 16 rows by all the tokens.  A code minus 32 is an int8; the scales
+// change every 16 elements, half an MFMA's depth, so each 32 elements are two
+// MFMAs with the other group's half of A zero (lanes 0-31 hold elements 0-15,
+// 32-63 the others), D = sc_a D_a + sc_b D_b in 32-bit integers (below 2^24,
+// exact as f32), and from there on as above: acc += xs D, and y += d acc per
+// unit (PROD: y += (d xs) D).  A stage ahead of its use, threads 0-127 turn
+// the quants of (row tid / 2, half tid % 2) into A fragments, 128-191 write the
+// row's scales and d, and all of them the stage's X fragments and scales.
+// 600 x 256 x 200: 11 us a call, 19 on the kernel above; 4800 x 512 x 200: 18 and 26.
+template <bool PROD>
+__global__ __launch_bounds__(256) void k_gemm_q6_small(Q8Args a) {
+  constexpr int NJ = Q6S / 16;
+  __shared__ __align__(16) uint8_t Aq[2][2][4][512];  // [buf][half][row tile][lane slot x 8 codes]
+  __shared__ __align__(16) int Sc[2][4][Q6S];         // [buf][group][row]
+  __shared__ __align__(16) float Dd[2][Q6S];
+  __shared__ __align__(16) float Xs[2][2][NJ][16];    // [buf][half][token tile][token]
+  __shared__ __align__(16) uint8_t Xb[2][2][NJ][512];
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int rows = a.rows, m0 = blockIdx.x * Q6S, n0 = blockIdx.y * Q6S;
+  const int stages = a.kpad / 64, kbs = a.kpad / 32;
+  const uint8_t *xq = (const uint8_t *)a.xq;
+  const int sr = tid < 128 ? tid >> 1 : tid - 128, sh = tid & 1;
+  const bool sq = tid < 128, ss = tid >= 128 && tid < 192;
+  const bool sok = m0 + sr < rows;
+  const uint8_t *srow = a.rec + (long)min(m0 + min(sr, Q6S - 1), rows - 1) * stages * 64;
+  u4_t c1 = {0, 0, 0, 0}, c2 = c1, xf;
+  u2_t hb = {0, 0};  // high bits, or the scales (x) and d (y)
+  float xsv = 0.f;
+  // this thread's 16 bytes of the stage's X fragments: fragment (half, token tile) tid / 32
+  const int xh = tid / (32 * NJ), xj = (tid >> 5) % NJ;
+  const uint8_t *xfp = xq + (long)((n0 >> 4) + xj) * kbs * 512 + xh * 512 + 16 * (tid & 31);
+  const float *xsp = a.xs + (long)((n0 >> 4) + ((tid >> 4) % NJ)) * kbs * 16 + (tid / (16 * NJ)) * 16 + (tid & 15);
+  auto load = [&](int s) {
+    const uint8_t *rp = srow + (long)s * 64;
+    if (sq) {
+      c1 = *(const u4_t *)(rp + 16);
+      c2 = *(const u4_t *)(rp + 32);
+      hb = *(const u2_t *)(rp + 48 + 8 * sh);
+    } else if (ss) {
+      hb = *(const u2_t *)rp;
     }
+    if (tid < 32 * NJ) xsv = xsp[(long)s * 32];
+    xf = *(const u4_t *)(xfp + (long)s * 1024);
+  };
+  auto store = [&](int buf) {
+    if (sq) {
+      // element 16 qq + i of half sh: its low 4 bits are nibble sh of byte i of
+      // c1 / c2, its high 2 bits at bits 2 i of dword qq of hb
+      uint8_t *fr = &Aq[buf][sh][sr >> 4][0];
+#pragma unroll
+      for (int j = 0; j < 4; j++) {  // codes 8 j .. 8 j + 7: lane slot (row % 16) + 16 j
+        uint32_t out[2];
+#pragma unroll
+        for (int e = 0; e < 2; e++) {
+          const int i0 = 8 * (j & 1) + 4 * e;
+          const uint32_t lo = ((j >> 1 ? c2 : c1)[i0 >> 2] >> (4 * sh)) & 0x0F0F0F0Fu;
+          const uint32_t b2 = (hb[j >> 1] >> (2 * i0)) & 0xFFu;
+          const uint32_t hi = (b2 | (b2 << 6) | (b2 << 12) | (b2 << 18)) & 0x03030303u;
+          out[e] = sok ? ((((lo | (hi << 4)) | 0x80808080u) - 0x20202020u) ^ 0x80808080u) : 0u;  // q - 32
+        }
+        *(uint2 *)(fr + ((sr & 15) + 16 * j) * 8) = make_uint2(out[0], out[1]);
+      }
+    } else if (ss) {
+#pragma unroll
+      for (int g = 0; g < 4; g++) Sc[buf][g][sr] = (int)(int8_t)(hb[0] >> (8 * g));
+      Dd[buf][sr] = sok ? h2f(hb[1]) : 0.f;
+    }
+    if (tid < 32 * NJ) Xs[buf][tid / (16 * NJ)][(tid >> 4) % NJ][tid & 15] = xsv;
+    *(u4_t *)&Xb[buf][xh][xj][16 * (tid & 31)] = xf;
+  };
+  f32x4_t y[NJ], acc[NJ];
+#pragma unroll
+  for (int jn = 0; jn < NJ; jn++) y[jn] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  const int rr0 = 16 * wave + 4 * (lane >> 4);  // this lane's rows rr0 .. rr0 + 3 of the block
+  auto compute = [&](int s) {
+    const int buf = s & 1;
+    const f32x4_t dd = *(const f32x4_t *)&Dd[buf][rr0];
+    if (!PROD && (s & 3) == 0) {
+#pragma unroll
+      for (int jn = 0; jn < NJ; jn++) acc[jn] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    }
+#pragma unroll
+    for (int h = 0; h < 2; h++) {
+      const long c = *(const long *)&Aq[buf][h][wave][lane * 8];
+      const long ca = lane < 32 ? c : 0, cb = lane < 32 ? 0 : c;  // groups 2 h and 2 h + 1
+      const i32x4_t sa = *(const i32x4_t *)&Sc[buf][2 * h][rr0], sb = *(const i32x4_t *)&Sc[buf][2 * h + 1][rr0];
+#pragma unroll
+      for (int jn = 0; jn < NJ; jn++) {
+        const long bx = *(const long *)&Xb[buf][h][jn][lane * 8];
+        const i32x4_t z = {0, 0, 0, 0};
+        const i32x4_t da = __builtin_amdgcn_mfma_i32_16x16x32_i8(ca, bx, z, 0, 0, 0);
+        const i32x4_t db = __builtin_amdgcn_mfma_i32_16x16x32_i8(cb, bx, z, 0, 0, 0);
+        const float xs = Xs[buf][h][jn][lane & 15];
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+          const float D = (float)(sa[r] * da[r] + sb[r] * db[r]);
+          if constexpr (PROD) y[jn][r] = fmaf(dd[r] * xs, D, y[jn][r]);
+          else acc[jn][r] = fmaf(xs, D, acc[jn][r]);
+        }
+      }
+    }
+    if (!PROD && (s & 3) == 3) {
+#pragma unroll
+      for (int jn = 0; jn < NJ; jn++)
+#pragma unroll
+        for (int r = 0; r < 4; r++) y[jn][r] = fmaf(dd[r], acc[jn][r], y[jn][r]);
+    }
+  };
+  load(0);
+  store(0);
+  __syncthreads();
+  for (int s = 0; s < stages; s++) {
+    const bool more = s + 1 < stages;
+    if (more) load(s + 1);
+    compute(s);
+    if (more) store((s + 1) & 1);
+    __syncthreads();
   }
-  return best;
+#pragma unroll
+  for (int jn = 0; jn < NJ; jn++) {
+    const int t = n0 + 16 * jn + (lane & 15);
+    if (t >= a.n) continue;
+#pragma unroll
+    for (int r = 0; r < 4; r++)
+      if (m0 + rr0 + r < rows) a.y[(long)t * rows + m0 + rr0 + r] = y[jn][r];
+  }
 }
-Q8Plan q8_plan(const Layout &L, int n, int num_cus) {
-  int k1 = 1, k2 = 1;
-  const double t1 = q8_split(L, 1, n, num_cus, k1), t2 = q8_split(L, 2, n, num_cus, k2);
-  Q8Plan p{};
-  p.nj = t2 < t1 - 1e-9 ? 2 : 1;
-  p.bn = 128 * p.nj;
-  p.ntiles = (n + p.bn - 1) / p.bn;
-  p.npad = p.ntiles * p.bn;
-  p.tiles = (L.rows + Q8_ROWS - 1) / Q8_ROWS;
-  p.ksplit = p.nj == 2 ? k2 : k1;
-  return p;
-}
+
 template <int FMT>
 void (*q8_kernel(int nj, int units))(Q8Args) {
   if (units == 1) return nj == 1 ? k_gemm_q8<FMT, 1, true> : k_gemm_q8<FMT, 2, true>;
   return nj == 1 ? k_gemm_q8<FMT, 1, false> : k_gemm_q8<FMT, 2, false>;
 }
-size_t up256(size_t v) { return (v + 255) & ~(size_t)255; }
-// Workspace: fragments, scales, thirds, partial products.
-struct Q8Bytes {
-  size_t xq, xs, xm, part;
-};
-Q8Bytes q8_bytes(const Q8Plan &p, const Layout &L, int n) {
-  const size_t tu = (size_t)(p.npad / 16) * L.units;
-  return {up256(tu * 8192), up256(tu * 512), up256(tu * 1024),
-          p.ksplit > 1 ? (size_t)p.ksplit * n * L.rows * 4 : 0};
-}
-
 }  // namespace
 
 size_t gemm_q8_workspace_bytes(const Layout &L, int n, int num_cus) {
-  const Q8Bytes b = q8_bytes(q8_plan(L, n, num_cus), L, n);
-  return b.xq + b.xs + b.xm + b.part + 256;
-}
-
-// A bound for every batch of up to n tokens.  A token tile's batches share
-// their block counts, so the shortest has the largest split of each tile size.
-size_t gemm_q8_workspace_bound(const Layout &L, int n, int num_cus) {
-  Q8Plan p{};
-  p.npad = (n + 255) / 256 * 256;
-  p.ksplit = 1;
-  const Q8Bytes b = q8_bytes(p, L, n);
-  size_t part = 0;
-  for (int n0 = 0; n0 < n; n0 += 128) {
-    int ks = 1;
-    for (int nj = 1; nj <= 2; nj++) {
-      int k = 1;
-      (void)q8_split(L, nj, n0 + 1, num_cus, k);
-      ks = std::max(ks, k);
-    }
-    if (ks > 1) part = std::max(part, (size_t)ks * std::min(n, n0 + 128) * L.rows * 4);
-  }
-  return b.xq + b.xs + b.xm + part + 256;
+  return q8_bytes(q8_plan(L.dtype, L.rows, L.units, n, num_cus), L.rows, L.units, n).total();
 }
 
 hipError_t launch_gemm_q8(const gq_weight *w, const float *X, int n, float *Y, void *workspace, int num_cus,
                           hipStream_t st) {
   const Layout &L = w->L;
   if (!w->gemm_raw) return hipErrorInvalidValue;
-  const Q8Plan p = q8_plan(L, n, num_cus);
-  const Q8Bytes bytes = q8_bytes(p, L, n);
+  const Q8Plan p = q8_plan(L.dtype, L.rows, L.units, n, num_cus);
+  const Q8Bytes bytes = q8_bytes(p, L.rows, L.units, n);
   char *ws = (char *)workspace;
   uint16_t *xq = (uint16_t *)ws;
   float *xs = (float *)(ws += bytes.xq);
@@ -488,8 +556,8 @@ hipError_t launch_gemm_q8(const gq_weight *w, const float *X, int n, float *Y, v
   float *part = (float *)(ws += bytes.xm);
   const long blocks = (long)(p.npad / 16) * L.units * 2, tiles = (long)p.tiles * p.ntiles * p.ksplit;
   if (blocks > 0x7fffffffL || tiles > 0x7fffffffL) return hipErrorInvalidValue;
-  hipLaunchKernelGGL(k_x_to_q8, dim3((unsigned)blocks), dim3(256), 0, st, X, n, p.npad, L.k, L.units, xq, xs,
-                     L.dtype == T_Q4_K ? xm : nullptr);
+  hipLaunchKernelGGL(p.small ? k_x_to_q8<true> : k_x_to_q8<false>, dim3((unsigned)blocks), dim3(256), 0, st, X, n,
+                     p.npad, L.k, L.units, xq, xs, L.dtype == T_Q4_K ? xm : nullptr);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
   Q8Args a{};
@@ -503,8 +571,12 @@ hipError_t launch_gemm_q8(const gq_weight *w, const float *X, int n, float *Y, v
   a.n = n;
   a.kpad = L.units * 256;
   a.ntiles = p.ntiles;
-  a.tiles = p.tiles;
   a.ksplit = p.ksplit;
+  if (p.small) {
+    hipLaunchKernelGGL(L.units == 1 ? k_gemm_q6_small<true> : k_gemm_q6_small<false>,
+                       dim3((unsigned)p.tiles, (unsigned)p.ntiles), dim3(256), 0, st, a);
+    return hipGetLastError();
+  }
   void (*kern)(Q8Args) = L.dtype == T_Q4_K ? q8_kernel<T_Q4_K>(p.nj, L.units) : q8_kernel<T_Q6_K>(p.nj, L.units);
   hipLaunchKernelGGL(kern, dim3((unsigned)tiles), dim3(512), 0, st, a);
   if ((e = hipGetLastError()) != hipSuccess || p.ksplit == 1) return e;

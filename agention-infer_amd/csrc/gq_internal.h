@@ -4,6 +4,7 @@
 #include <stddef.h>
 #include <stdint.h>
 
+#include "gq_gemm_plan.h"
 #include "gq_layout.h"
 
 // The public handle (opaque in gq.h).
@@ -217,7 +218,6 @@ size_t gemm_workspace_bytes(const gq_weight *w, int n, int mode, int num_cus);
 size_t gemm_workspace_bound(const gq_weight *w, int n, int num_cus);  // any mode, up to n tokens
 // Its int8 mode (Q4_K, Q6_K).
 size_t gemm_q8_workspace_bytes(const Layout &L, int n, int num_cus);
-size_t gemm_q8_workspace_bound(const Layout &L, int n, int num_cus);
 hipError_t launch_gemm_q8(const gq_weight *w, const float *X, int n, float *Y, void *workspace, int num_cus,
                           hipStream_t st);
 // y[i] = sum_s part[s][i], s in order, i < count.

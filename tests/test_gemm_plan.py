@@ -1,0 +1,72 @@
+"""The batched product's launch rules on the CPU, against measured times."""
+import os
+import subprocess
+
+import pytest
+
+from gemm_shapes import INT8_KERNELS, Q4_K, Q6_K
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+
+
+@pytest.fixture(scope="module")
+def ask(tmp_path_factory):
+    exe = tmp_path_factory.mktemp("plan") / "gemm_plan"
+    r = subprocess.run(["g++", "-O1", "-std=c++17", "-Wall", "-Wextra", "-Werror",
+                        "-I", os.path.join(ROOT, "agention-infer_amd", "csrc"),
+                        os.path.join(ROOT, "tests", "cpp", "gemm_plan.cpp"), "-o", str(exe)],
+                       capture_output=True, text=True)
+    assert r.returncode == 0, r.stderr
+
+    def run(lines):
+        r = subprocess.run([str(exe)], input="\n".join(lines) + "\n", capture_output=True, text=True, timeout=60)
+        assert r.returncode == 0
+        out = [[int(v) for v in line.split()] for line in r.stdout.splitlines()]
+        assert len(out) == len(lines)
+        return out
+    return run
+
+
+def units(k):
+    return (k + 255) // 256
+
+
+# Q6_K int8 calls: (rows, k, tokens, us on the 64 x 64 blocks, us on the
+# 160-row ones with their K split).
+Q6_TIMES = [
+    (64, 256, 2, 11.2, 15.9), (133, 256, 200, 11.1, 19.7), (600, 256, 200, 11.3, 19.2),
+    (2400, 256, 128, 11.4, 20.3), (4800, 256, 300, 13.9, 21.1), (9000, 256, 512, 26.1, 21.5),
+    (14336, 256, 64, 11.4, 18.1), (18944, 256, 384, 33.3, 25.8), (133, 512, 2, 12.7, 16.5),
+    (1200, 512, 512, 15.5, 22.8), (4800, 512, 200, 17.5, 26.1), (9000, 512, 384, 29.2, 26.7),
+    (9000, 512, 700, 43.6, 31.9), (2400, 768, 700, 25.6, 35.6), (4800, 768, 300, 25.0, 34.3),
+    (9000, 768, 700, 58.2, 42.7), (14336, 768, 200, 34.6, 34.9), (64, 1024, 2, 20.6, 16.2),
+    (600, 1024, 16, 21.5, 17.1), (2400, 1024, 300, 23.8, 27.4), (4800, 1024, 300, 30.4, 35.1),
+    (9000, 1024, 512, 55.6, 44.2), (9000, 1280, 300, 44.2, 50.0), (133, 2048, 64, 38.1, 19.5),
+    (3584, 2048, 512, 52.7, 50.4), (3584, 3072, 64, 55.7, 30.0),
+]
+
+
+def test_q6_small_rule(ask):
+    """The rule takes the faster of the two kernels wherever they differ by
+    more than the estimates can tell."""
+    got = ask([f"q8 {Q6_K} {r} {units(k)} {n}" for r, k, n, _, _ in Q6_TIMES])
+    for (r, k, n, small, big), g in zip(Q6_TIMES, got):
+        taken, other = (small, big) if g[0] else (big, small)
+        assert taken <= 1.05 * other, f"{r} x {k} at {n} tokens: takes {taken} us, the other {other}"
+
+
+def test_int8_test_shapes_take_their_kernel(ask):
+    got = ask([f"q8 {t} {r} {units(k)} {n}" for t, r, k, n, _ in INT8_KERNELS])
+    for (t, r, k, n, kernel), g in zip(INT8_KERNELS, got):
+        assert kernel == ("small" if g[0] else 128 * g[1]), f"dtype {t}, {r} x {k} at {n} tokens: {g}"
+
+
+def test_q8_workspace_bound(ask):
+    """The bound for batches of up to n tokens covers each of them."""
+    shapes = [(t, r, u) for t in (Q4_K, Q6_K) for r, u in
+              ((1, 1), (133, 2), (91, 4), (512, 14), (3584, 74), (18944, 14), (161, 6), (40000, 3))]
+    for t, r, u in shapes:
+        got = ask([f"q8 {t} {r} {u} {n}" for n in range(1, 700, 13)])
+        bytes_ = [g[3] for g in got]
+        for i, g in enumerate(got):
+            assert max(bytes_[:i + 1]) <= g[4]

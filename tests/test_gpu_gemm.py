@@ -17,6 +17,7 @@ import numpy as np
 import pytest
 
 import gq_synth as syn
+from gemm_shapes import INT8_KERNELS
 
 pytestmark = pytest.mark.gpu
 
@@ -155,6 +156,44 @@ def test_gemm_int8_tiles(backend, orc, dtype, rows, k, n):
         sc, q = orc.quantize_q8_32(X[t])
         Xq[t, :q.size] = q.astype(np.float64) * np.repeat(sc.view(np.float16).astype(np.float64), 32)[:q.size]
     check(Y, Xq[:, :k] @ Wf.T, "int8 vs same-operand fp64")
+
+
+def int8_ref(orc, dtype, w, X):
+    """The int8 mode's product in float64: exact dequant times the Q8 pack."""
+    n, k = X.shape
+    Xq = np.zeros((n, k), np.float64)
+    for t in range(n):
+        sc, q = orc.quantize_q8_32(X[t])
+        Xq[t] = q.astype(np.float64) * np.repeat(sc.view(np.float16).astype(np.float64), 32)[:k]
+    return Xq @ orc.dequant_rows(dtype, w, k).astype(np.float64).T
+
+
+@pytest.mark.parametrize("dtype,rows,k,n,kernel", INT8_KERNELS)
+def test_gemm_int8_kernels(backend, orc, dtype, rows, k, n, kernel):
+    """Each kernel of the int8 mode at the edges of its tiles.  Every integer
+    in it is exact, so per token only the roundings of up to 8 units + 2 f32
+    sums and the reference's f32 weights are left: 2^-24 each of terms of the
+    result's size, below 1e-6 of it together."""
+    import gq
+    import torch
+    say(f"gemm int8 {kernel} dtype={dtype} rows={rows} k={k} n={n}")
+    rng = np.random.default_rng(rows + k + n)
+    w = syn.make_blocks(dtype, rows, k, seed=rows + n)
+    if dtype == Q6_K:  # scales over all of int8
+        b = w.reshape(rows, -1, 210)
+        b[..., 192:208] = rng.integers(-128, 128, b[..., 192:208].shape, dtype=np.int8).view(np.uint8)
+    X = syn.make_x(k, seed=n, batch=n)
+    ref = int8_ref(orc, dtype, w, X)
+    size = np.sqrt(np.mean(ref ** 2, axis=1) + 1e-300)
+    h = backend.upload_weight(dtype, w, k, rows)
+    for off in (0, 1):  # X aligned, and to 4 bytes only
+        buf = torch.zeros(n * k + 1, device="cuda")
+        buf[off:off + n * k] = torch.from_numpy(X).cuda().view(-1)
+        Y = h.launch_only_batch(buf[off:off + n * k].view(n, k), mode=gq.GQ_GEMM_INT8).cpu().numpy()
+        err = np.sqrt(np.mean((Y - ref) ** 2, axis=1)) / size
+        say(f"  worst token {err.max():.3g}")
+        # (one row: the result may be small beside its terms)
+        assert err.max() <= (1e-6 if rows > 1 else 1e-5)
 
 
 def test_gemm_full_config(backend, orc):
