@@ -331,37 +331,49 @@ struct StreamWs {
   hipStream_t st;
   void *p;
   size_t bytes;
+  size_t denied;  // the smallest room that could not be had
 };
 std::vector<StreamWs> g_stream_ws;  // guarded by g_mu
 std::vector<void *> g_retired_ws;   // superseded workspaces, guarded by g_mu
 
-int stream_workspace(hipStream_t st, size_t bytes, void **out) {
+// `bytes` of workspace on st; if it has to grow, or is smaller than `room`, it
+// becomes `room` bytes if these are to be had.
+int stream_workspace(hipStream_t st, size_t bytes, size_t room, void **out) {
   std::lock_guard<std::mutex> lk(g_mu);
   int dev = 0;
   (void)hipGetDevice(&dev);
   StreamWs *ws = nullptr;
   for (StreamWs &w : g_stream_ws)
     if (w.dev == dev && w.st == st) ws = &w;
-  if (ws && ws->bytes >= bytes) {
+  const size_t held = ws ? ws->bytes : 0;
+  if (held >= std::max(bytes, room)) {
     *out = ws->p;
     return GQ_OK;
   }
-  if (stream_capturing(st))
-    return fail(GQ_EINVAL,
-                "stream workspace of %zu bytes needed under graph capture (the stream holds %zu): "
-                "make one call of at least this size on the stream before capturing",
-                bytes, ws ? ws->bytes : (size_t)0);
-  void *p = nullptr;
-  if (hipMalloc(&p, bytes) != hipSuccess)
-    return fail(GQ_ENOMEM, "workspace of %zu bytes: hipMalloc failed", bytes);
-  if (ws) {
-    g_retired_ws.push_back(ws->p);
-    ws->p = p;
-    ws->bytes = bytes;
-  } else {
-    g_stream_ws.push_back(StreamWs{dev, st, p, bytes});
+  if (stream_capturing(st)) {
+    if (held < bytes)
+      return fail(GQ_EINVAL,
+                  "stream workspace of %zu bytes needed under graph capture (the stream holds %zu): "
+                  "make one call of at least this size on the stream before capturing",
+                  bytes, held);
+    *out = ws->p;
+    return GQ_OK;
   }
-  *out = p;
+  StreamWs now = ws ? *ws : StreamWs{dev, st, nullptr, 0, SIZE_MAX};
+  const bool ok = gq::take_workspace(now.p, now.bytes, now.denied, bytes, room, [](size_t n) -> void * {
+    void *p = nullptr;
+    if (hipMalloc(&p, n) == hipSuccess) return p;
+    (void)hipGetLastError();  // (the launch checks read it)
+    return nullptr;
+  });
+  if (!ok) return fail(GQ_ENOMEM, "workspace of %zu bytes: hipMalloc failed", bytes);
+  if (!ws) {
+    g_stream_ws.push_back(now);
+  } else {
+    if (now.p != ws->p) g_retired_ws.push_back(ws->p);
+    *ws = now;
+  }
+  *out = now.p;
   return GQ_OK;
 }
 }  // namespace
@@ -407,7 +419,7 @@ int moe_ffn(const gq_weight *gate, const gq_weight *up, const gq_weight *down, i
     if (g_dev.device < 0 || g_dev.device >= MAX_DEVICES || !g_scratch_dev[g_dev.device])
       return fail(GQ_ENODEV, "gq_moe_ffn_noalloc: no scratch on device %d", g_dev.device);
     wsp = (char *)g_scratch_dev[g_dev.device];
-  } else if ((rc = stream_workspace((hipStream_t)stream, ws, (void **)&wsp))) {
+  } else if ((rc = stream_workspace((hipStream_t)stream, ws, ws, (void **)&wsp))) {
     return rc;
   }
   gq::MoeArgs a{};
@@ -676,7 +688,7 @@ int gq_gemm(const gq_weight *w, const float *X_dev, int n, float *Y_dev, int mod
   if (n < 0) return fail(GQ_EINVAL, "negative batch");
   if (n == 0 || w->L.rows == 0) return GQ_OK;
   if (mode != GQ_GEMM_BF16 && mode != GQ_GEMM_INT8) return fail(GQ_EINVAL, "bad gemm mode %d", mode);
-  size_t ws = gq::gemm_workspace_bytes(w, n, mode, g_dev.num_cus);
+  const size_t ws = gq::gemm_workspace_bytes(w, n, mode, g_dev.num_cus);
   if (ws == (size_t)-1)
     return fail(GQ_EDTYPE, "gq_gemm: %s weights not supported in %s mode", type_name(w->L.dtype),
                 mode == GQ_GEMM_BF16 ? "bf16" : "int8");
@@ -686,9 +698,9 @@ int gq_gemm(const gq_weight *w, const float *X_dev, int n, float *Y_dev, int mod
   }
   // An eager call takes room for every call of up to n tokens, so that these
   // may be captured afterwards.
-  if (!stream_capturing((hipStream_t)stream)) ws = std::max(ws, gq::gemm_workspace_bound(w, n, g_dev.num_cus));
+  const size_t room = std::max(ws, gq::gemm_workspace_bound(w, n, g_dev.num_cus));
   void *wsp = nullptr;
-  if (ws && (rc = stream_workspace((hipStream_t)stream, ws, &wsp))) return rc;
+  if ((rc = stream_workspace((hipStream_t)stream, ws, room, &wsp))) return rc;
   hipError_t e = gq::launch_gemm(w, X_dev, n, Y_dev, mode, wsp, ws, g_dev.num_cus,
                                  (hipStream_t)stream);
   if (e != hipSuccess) return fail(GQ_EHIP, "gemm launch failed: %s", hipGetErrorString(e));

@@ -693,16 +693,27 @@ size_t gemm_workspace_bytes(const gq_weight *w, int n, int mode, int num_cus) {
   return gemm_q8_workspace_bytes(w->L, n, num_cus);
 }
 
-// Bytes that serve any call on w of up to n tokens, in either mode.  (A
-// shorter batch has fewer blocks and so may split K further, into more
-// partial products than a longer one.)
+// Bytes that serve any call on w of up to gemm_room_tokens(n) tokens, in either
+// mode, and the X of any bf16 call of up to n rounded up to 512.  (A shorter
+// batch has fewer blocks and so may split K further, into more partial
+// products than a longer one.)  The weight keeps the last answer: the search
+// costs a microsecond or two, and most calls ask the same again.
 size_t gemm_workspace_bound(const gq_weight *w, int n, int num_cus) {
-  size_t b = gemm_workspace_bytes(w, n, GQ_GEMM_BF16, num_cus);
-  if (n > GEMM_QUAD_MAX) b = std::max(b, gemm_workspace_bytes(w, GEMM_QUAD_MAX, GQ_GEMM_BF16, num_cus));
-  for (int m = GEMM_NPAD; m < n; m += GEMM_NPAD)
-    b = std::max(b, gemm_workspace_bytes(w, m, GQ_GEMM_BF16, num_cus));
-  if (w->L.dtype == T_Q4_K || w->L.dtype == T_Q6_K) 
-    b = std::max(b, q8_bytes_bound(w->L.rows, w->L.units, n, num_cus));
+  const long nr = gemm_room_tokens(n);
+  uint64_t *memo = const_cast<uint64_t *>(&w->gemm_room);  // nr / 256 << 41 | bytes / 256
+  const uint64_t m = __atomic_load_n(memo, __ATOMIC_RELAXED);
+  if (m >> 41 == (uint64_t)nr / 256) return (size_t)(m & ((1ull << 41) - 1)) * 256;
+  if (nr > 0x7fffff00) return 0;
+  const int nmax = (int)nr;
+  size_t b = std::max(gemm_workspace_bytes(w, nmax, GQ_GEMM_BF16, num_cus),
+                      gemm_workspace_bytes(w, GEMM_QUAD_MAX, GQ_GEMM_BF16, num_cus));
+  for (int t = GEMM_NPAD; t < nmax; t += GEMM_NPAD)
+    b = std::max(b, gemm_workspace_bytes(w, t, GQ_GEMM_BF16, num_cus));
+  if (nmax < 512) b = std::max(b, gemm_x_elems(w->L.units, 512, false) * 2 + 256);
+  if (w->L.dtype == T_Q4_K || w->L.dtype == T_Q6_K)
+    b = std::max(b, q8_bytes_bound(w->L.rows, w->L.units, nmax, num_cus));
+  b = (b + 255) & ~(size_t)255;
+  if (b >> 8 < 1ull << 41) __atomic_store_n(memo, (uint64_t)nr / 256 << 41 | b / 256, __ATOMIC_RELAXED);
   return b;
 }
 

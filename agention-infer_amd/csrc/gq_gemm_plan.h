@@ -8,6 +8,40 @@
 
 namespace gq {
 
+// ----------------------------------------------------------- workspace
+// The batch that an eager call of n tokens takes workspace for: n rounded up
+// to 256 and, past 1024, to a quarter of a power of two.  Superseded workspaces
+// are kept, so a growing batch must not grow its workspace with every token:
+// the sizes are a third or more apart, and the kept ones at most 3 times the
+// last.
+inline long gemm_room_tokens(int n) {
+  long step = 256;
+  while (4 * step < n) step *= 2;
+  return (n + step - 1) / step * step;
+}
+
+// A workspace of `held` bytes (at `p`), a call that needs `need` of them and
+// would take `room`: what to use.  The room is for other calls to come, so
+// where alloc(room) gives nothing the call goes on with its own bytes, and
+// that much room is not asked for again (`denied`).  False: not even those.
+template <class Alloc>
+bool take_workspace(void *&p, size_t &held, size_t &denied, size_t need, size_t room, Alloc alloc) {
+  if (room > held && room < denied) {
+    if (void *q = alloc(room)) {
+      p = q;
+      held = room;
+    } else {
+      denied = room;
+    }
+  }
+  if (need <= held) return true;
+  void *q = alloc(need);
+  if (!q) return false;
+  p = q;
+  held = need;
+  return true;
+}
+
 // ----------------------------------------------------------- int8 mode
 // (gq_gemm_q8.hip.)  small: 64 x 64 blocks, no K split; else 160 rows x 128 nj
 // tokens.

@@ -14,7 +14,8 @@ struct gq_weight {
   uint16_t *d;       // per-unit f16 scales (Q6_K, IQ3_XXS), or nullptr
   size_t ggml_bytes; // size of the tensor in ggml block order
   int device;
-  uint8_t *gemm_raw = nullptr;  // per-stage records for the bf16 GEMM (made on first use)
+  uint8_t *gemm_raw = nullptr;  // per-stage records for the GEMM (made on first use)
+  uint64_t gemm_room = 0;       // gemm_workspace_bound's last answer (atomic access)
 };
 
 namespace gq {
@@ -215,7 +216,7 @@ hipError_t launch_quantize_row_q8k(const float *x, long n, float *d, int8_t *qs,
 hipError_t launch_gemm(const gq_weight *w, const float *X, int n, float *Y, int mode,
                        void *workspace, size_t ws_bytes, int num_cus, hipStream_t st);
 size_t gemm_workspace_bytes(const gq_weight *w, int n, int mode, int num_cus);
-size_t gemm_workspace_bound(const gq_weight *w, int n, int num_cus);  // any mode, up to n tokens
+size_t gemm_workspace_bound(const gq_weight *w, int n, int num_cus);  // any mode, up to n tokens and some
 // Its int8 mode (Q4_K, Q6_K).
 size_t gemm_q8_workspace_bytes(const Layout &L, int n, int num_cus);
 hipError_t launch_gemm_q8(const gq_weight *w, const float *X, int n, float *Y, void *workspace, int num_cus,

@@ -121,7 +121,8 @@ int gq_dequant_rows_host(const gq_weight *w, int row0, int nrows, float *out_hos
  * that first call was made before and the stream's workspace already holds
  * the call's bytes; otherwise it fails with GQ_EINVAL and records nothing.
  * (An eager call takes room for every call on its weight of up to n tokens,
- * in either mode.)
+ * n rounded up, in either mode; where that much memory is not to be had, it
+ * takes its own bytes and goes on.)
  * Workspaces are never freed while the process runs, so a captured graph
  * stays valid when later, larger calls grow the stream's workspace. */
 int gq_gemm(const gq_weight *w, const float *X_dev, int n, float *Y_dev, int mode, void *stream);

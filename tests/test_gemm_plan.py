@@ -70,3 +70,32 @@ def test_q8_workspace_bound(ask):
         bytes_ = [g[3] for g in got]
         for i, g in enumerate(got):
             assert max(bytes_[:i + 1]) <= g[4]
+
+
+def test_room_tokens(ask):
+    """A batch that grows token by token takes few workspaces, and the kept
+    ones come to at most 3 times the last."""
+    sizes = [g[0] for g in ask([f"room {n}" for n in range(1, 9000)])]
+    assert all(n <= s <= max(256, 3 * n // 2 + 256) for n, s in enumerate(sizes, 1))
+    steps = sorted(set(sizes))
+    assert sizes == sorted(sizes) and len(steps) <= 12
+    for i in range(1, len(steps)):
+        assert sum(steps[:i]) <= 3 * steps[i]
+
+
+def test_take_workspace(ask):
+    """Room beyond a call's own bytes is taken where it can be had, and the
+    call goes on without where not (and does not ask again each time)."""
+    big = 1 << 60
+    cases = {
+        (0, big, 10, 50, 100): (1, 50, big, 1),   # room to be had
+        (0, big, 10, 50, 20): (1, 10, 50, 2),     # only its own bytes
+        (10, 50, 10, 50, 20): (1, 10, 50, 0),     # held, the room refused before
+        (10, big, 10, 50, 20): (1, 10, 50, 1),    # held, the room refused now
+        (10, 50, 10, 40, 45): (1, 40, 50, 1),     # less room than was refused
+        (10, 50, 30, 60, 35): (1, 30, 50, 1),     # growth, room known to be refused
+        (0, big, 10, 50, 5): (0, 0, 50, 2),       # not even that
+        (60, big, 10, 50, 100): (1, 60, big, 0),  # held
+    }
+    got = ask(["take " + " ".join(map(str, c)) for c in cases])
+    assert [tuple(g) for g in got] == list(cases.values())

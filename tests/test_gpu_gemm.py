@@ -305,6 +305,51 @@ def test_gemm_capture_of_shorter_batches(backend, mode):
             assert torch.equal(Y[:n], ref), f"n {n} replay {i}"
 
 
+def test_gemm_growing_batch_keeps_little(backend):
+    """Batches that grow on one stream: the workspaces that later ones
+    supersede are kept, so only a few sizes may be taken."""
+    import torch
+    rows, k = 18944, 3584
+    h = backend.upload_weight(Q4_K, syn.make_blocks(Q4_K, rows, k, seed=75), k, rows)
+    X = torch.from_numpy(syn.make_x(k, seed=76, batch=512)).cuda()
+    Y = torch.zeros((512, rows), device="cuda")
+    s = torch.cuda.Stream()
+    h.launch_only_batch(X[:1], Y_dev=Y[:1])  # (the weight's records)
+    torch.cuda.synchronize()
+    free = torch.cuda.mem_get_info()[0]
+    for n in range(1, 513, 7):
+        h.launch_only_batch(X[:n], Y_dev=Y[:n], mode=n % 2, stream=s.cuda_stream)
+    s.synchronize()
+    kept = free - torch.cuda.mem_get_info()[0]
+    say(f"kept {kept / 1e6:.1f} MB")
+    assert kept <= 200e6
+
+
+@pytest.mark.parametrize("mode,rows,k,n0,n", [(1, 600, 512, 1, 256), (1, 600, 512, 300, 512), (0, 41000, 256, 1, 512)])
+def test_gemm_capture_of_longer_batches(backend, mode, rows, k, n0, n):
+    """A warm-up with fewer tokens leaves room for the longer ones that share
+    its padding."""
+    import torch
+    h = backend.upload_weight(Q4_K, syn.make_blocks(Q4_K, rows, k, seed=77), k, rows)
+    X = torch.from_numpy(syn.make_x(k, seed=78, batch=n)).cuda()
+    Y = torch.zeros((n, rows), device="cuda")
+    s = torch.cuda.Stream()
+    torch.cuda.synchronize()
+    h.launch_only_batch(X[:n0], mode=mode, Y_dev=Y[:n0], stream=s.cuda_stream)
+    s.synchronize()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g, stream=s):
+        h.launch_only_batch(X, mode=mode, Y_dev=Y, stream=s.cuda_stream)
+    ref = h.launch_only_batch(X, mode=mode)
+    torch.cuda.synchronize()
+    for i in range(2):
+        Y.zero_()
+        torch.cuda.synchronize()
+        g.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(Y, ref), f"replay {i}"
+
+
 def test_gemm_capture_survives_workspace_growth(backend):
     """A HIP graph captured around gq_gemm keeps its workspace: a later,
     larger call on the same stream grows the stream's workspace without
