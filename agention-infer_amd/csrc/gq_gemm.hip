@@ -603,27 +603,6 @@ int gemm_ksplit(int tiles, int stages, int num_cus) {
   return best;
 }
 
-// K split of the short-batch kernel's launch of `tiles` row tiles and Tq
-// quads per row: the least estimated time, in units of one quad's work of a
-// block (one block per CU; about 4.8 us for Q6_K at 16 tokens): half a unit
-// to start, and a reduction launch when K is split.  Measured, us a call: 3584 x
-// 18944 Q6_K at 37 tokens (32 tiles) 107 unsplit, 50 in 3, 36 in 5, 32 in 8, 41
-// in 10 (a second round); 18944 x 3584 Q4_K (170 tiles) 28 unsplit, 35 in 2;
-// 8192 x 2048 Q8_0 at 8 tokens (74 tiles) 15.8 unsplit, 14.5 in 2.
-int gemm_quad_ksplit(int tiles, int Tq, int num_cus) {
-  int best = 1;
-  double best_t = 1e30;
-  for (int ks = 1; ks <= std::min(Tq, 16); ks++) {
-    const int rounds = (tiles * ks + num_cus - 1) / num_cus;
-    const double t = rounds * (0.5 + (Tq + ks - 1) / ks) + (ks > 1 ? 0.7 + 0.05 * ks : 0.0);
-    if (t < best_t - 1e-9) {
-      best_t = t;
-      best = ks;
-    }
-  }
-  return best;
-}
-
 namespace {
 struct GemmPlan {
   bool quad;                        // gq_gemm_quad.hip's kernel
@@ -636,10 +615,15 @@ GemmPlan gemm_plan(const gq_weight *const *ws, int count, int n, int num_cus) {
   p.tbn = p.quad ? 16 * gemm_quad_nt(n) : BN;
   p.ntiles = (n + p.tbn - 1) / p.tbn;
   int mt = 0;
-  for (int i = 0; i < count; i++) mt += (ws[i]->L.rows + p.tbm - 1) / p.tbm;
+  long rows = 0;
+  for (int i = 0; i < count; i++) {
+    mt += (ws[i]->L.rows + p.tbm - 1) / p.tbm;
+    rows += ws[i]->L.rows;
+  }
   p.tiles = mt * p.ntiles;
-  const int U = ws[0]->L.units, parts = p.quad ? (U + 3) / 4 : U * 4;
-  p.ksplit = p.quad ? gemm_quad_ksplit(p.tiles, parts, num_cus) : gemm_ksplit(p.tiles, parts, num_cus);
+  const int U = ws[0]->L.units;
+  p.ksplit = p.quad ? gemm_quad_ksplit(ws[0]->L.dtype, p.tiles, rows, U, n, num_cus)
+                    : gemm_ksplit(p.tiles, U * 4, num_cus);
   return p;
 }
 }  // namespace
@@ -697,7 +681,7 @@ size_t gemm_workspace_bytes(const gq_weight *w, int n, int mode, int num_cus) {
 // mode, and the X of any bf16 call of up to n rounded up to 512.  (A shorter
 // batch has fewer blocks and so may split K further, into more partial
 // products than a longer one.)  The weight keeps the last answer: the search
-// costs a microsecond or two, and most calls ask the same again.
+// costs some tens of microseconds, and most calls ask the same again.
 size_t gemm_workspace_bound(const gq_weight *w, int n, int num_cus) {
   const long nr = gemm_room_tokens(n);
   uint64_t *memo = const_cast<uint64_t *>(&w->gemm_room);  // nr / 256 << 41 | bytes / 256
@@ -705,9 +689,10 @@ size_t gemm_workspace_bound(const gq_weight *w, int n, int num_cus) {
   if (m >> 41 == (uint64_t)nr / 256) return (size_t)(m & ((1ull << 41) - 1)) * 256;
   if (nr > 0x7fffff00) return 0;
   const int nmax = (int)nr;
-  size_t b = std::max(gemm_workspace_bytes(w, nmax, GQ_GEMM_BF16, num_cus),
-                      gemm_workspace_bytes(w, GEMM_QUAD_MAX, GQ_GEMM_BF16, num_cus));
-  for (int t = GEMM_NPAD; t < nmax; t += GEMM_NPAD)
+  size_t b = 0;
+  for (int t = 1; t <= GEMM_QUAD_MAX; t++)  // (a split per batch)
+    b = std::max(b, gemm_workspace_bytes(w, t, GQ_GEMM_BF16, num_cus));
+  for (int t = GEMM_NPAD; t <= nmax; t += GEMM_NPAD)
     b = std::max(b, gemm_workspace_bytes(w, t, GQ_GEMM_BF16, num_cus));
   if (nmax < 512) b = std::max(b, gemm_x_elems(w->L.units, 512, false) * 2 + 256);
   if (w->L.dtype == T_Q4_K || w->L.dtype == T_Q6_K)

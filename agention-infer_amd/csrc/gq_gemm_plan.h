@@ -42,6 +42,55 @@ bool take_workspace(void *&p, size_t &held, size_t &denied, size_t need, size_t 
   return true;
 }
 
+// ----------------------------------------------------------- bf16 mode
+// (gq_gemm_quad.hip.)  Batches of up to GEMM_QUAD_MAX tokens in blocks of
+// GEMM_QUAD_ROWS weight rows by all the tokens; a step of its K loop is a quad of
+// units.
+constexpr int GEMM_QUAD_MAX = 128, GEMM_QUAD_ROWS = 112;
+
+// Token tiles of a batch of n <= 128: 1, 2, 3, 4, 6 or 8.
+inline int gemm_quad_nt(int n) {
+  const int t = (n + 15) / 16;
+  return t <= 4 ? t : t <= 6 ? 6 : 8;
+}
+
+// Estimated time of a short batch's call, us, on `tiles` row tiles (`rows` rows
+// in all) with K in ks parts: rounds of blocks (one a CU), each a start, its
+// quads' dequant and MFMAs, and what of their weights' way from HBM these do not
+// cover (longer the more of the CUs load at once); a split adds the reduction's
+// launch and writes and reads ks partial products.  The constants are those
+// that choose best, here and in gemm_quad_faster, over 9860 measured calls of 1
+// to 128 tokens on 64 x 256 to 128256 x 2048 weights; of the times themselves
+// they miss 11% on average.
+inline double gemm_quad_time(int dtype, int tiles, long rows, int units, int n, int ks, int num_cus) {
+  const int nt = gemm_quad_nt(n), quads = ((units + 3) / 4 + ks - 1) / ks;
+  const double rounds = (double)(((long)tiles * ks + num_cus - 1) / num_cus), fill = tiles * ks / (rounds * num_cus);
+  const double bits = dtype == 12 ? 4.5 : dtype == 13 ? 5.5 : dtype == 14 ? 6.5625 : 8.5;
+  const double hbm = fill * num_cus * GEMM_QUAD_ROWS * 256 * bits / 8 / 4.7e6;  // a unit of every block
+  const double step = (dtype == 12 ? 2.85 : dtype == 8 ? 2.7 : 3.4) + 0.75 * nt;
+  const double out = (double)rows * n * 8e-6 / 4.5;  // a result written and read
+  return 4.7 + rounds * (0.9 + 0.11 * hbm * std::min(4 * quads, units) + step * quads) +
+         (ks > 1 ? 2.85 + 1.1 * ks * out : 0.0) + 0.58 * out;
+}
+
+// The K split (over quads) of such a call: the least estimated time.  Measured
+// unsplit / in 2, us a call: 3584 x 2048 Q8_0 at 128 tokens 22.6 / 19.1, 9000 x
+// 2048 Q4_K at 128 23.5 / 24.2, 14336 x 2048 Q4_K at 128 24.8 / 28.5, 65536 x
+// 3584 Q6_K at 64 93.4 / 103.8 (the partial products' traffic); 3584 x 18944
+// Q6_K at 37 107 unsplit, 50 in 3, 36 in 5, 32 in 8, 41 in 10 (a second round).
+inline int gemm_quad_ksplit(int dtype, int tiles, long rows, int units, int n, int num_cus) {
+  int best = 1;
+  double best_t = 1e30;
+  for (int ks = 1; ks <= std::min((units + 3) / 4, 16); ks++) {
+    const double t = gemm_quad_time(dtype, tiles, rows, units, n, ks, num_cus);
+    if (t < best_t - 1e-9) {
+      best_t = t;
+      best = ks;
+    }
+  }
+  return best;
+}
+
 // ----------------------------------------------------------- int8 mode
 // (gq_gemm_q8.hip.)  small: 64 x 64 blocks, no K split; else 160 rows x 128 nj
 // tokens.

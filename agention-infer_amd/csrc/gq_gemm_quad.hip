@@ -300,12 +300,6 @@ void (*quad_kernel(int nt))(GemmArgs) {
 
 }  // namespace
 
-// Token tiles of a batch of n <= 128: 1, 2, 3, 4, 6 or 8.
-int gemm_quad_nt(int n) {
-  const int t = (n + 15) / 16;
-  return t <= 4 ? t : t <= 6 ? 6 : 8;
-}
-
 hipError_t launch_x_to_quad(const float *X, int n, int k, uint16_t *xb, hipStream_t st) {
   const int Tq = (k + 1023) / 1024, npad = 16 * gemm_quad_nt(n);
   const long threads = (long)(npad / 16) * Tq * 32 * 64;

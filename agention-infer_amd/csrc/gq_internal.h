@@ -259,10 +259,7 @@ struct GemmArgs {
 // for longer ones X fragments must cover n rounded up to GEMM_NPAD (the
 // 256-token tile).
 constexpr int GEMM_NPAD = 256;
-constexpr int GEMM_QUAD_MAX = 128;
-constexpr int GEMM_QUAD_ROWS = 112;  // weight rows per block of that kernel
 bool gemm_uses_quad(const gq_weight *const *ws, int count, int n);
-int gemm_quad_nt(int n);
 size_t gemm_x_elems(int units, int n, bool quad);
 hipError_t launch_x_to_quad(const float *X, int n, int k, uint16_t *xb, hipStream_t st);
 hipError_t launch_gemm_quad(const GemmArgs &a, int fmt, int blocks, hipStream_t st);

@@ -17,6 +17,7 @@
 // activations: bf16 of the fp32 values), accumulation fp32; everything
 // else is fp32 as on the CPU path.
 #include <algorithm>
+#include <vector>
 
 #include "gq_device.h"
 #include "gq_internal.h"
@@ -585,12 +586,22 @@ __global__ __launch_bounds__(512) void k_attn_prefill(const float *q, const uint
 // ------------------------------------------------------------------ host
 static int round_up(int v, int m) { return (v + m - 1) / m * m; }
 
-// The largest partial buffer of any launch of a pass of up to nmax tokens
-// (the K split depends on the batch's tiles, of 16 tokens for a short batch).
+// The largest partial buffer of any launch of a pass of up to nmax tokens (the K
+// split depends on the batch, past GEMM_QUAD_MAX tokens on its token tiles).
 size_t prefill_part_floats(const DecodeLaunch &m, int nmax, int num_cus) {
+  std::vector<int> layers;  // one of each set of shapes
+  for (int L = 0; L < m.n_layers; L++) {
+    auto alike = [&](int l) {
+      for (const gq_weight *const *w : {m.wq, m.wk, m.wv, m.wo, m.wgate, m.wup, m.wdown})
+        if (w[L]->L.dtype != w[l]->L.dtype || w[L]->L.rows != w[l]->L.rows || w[L]->L.units != w[l]->L.units)
+          return false;
+      return true;
+    };
+    if (std::none_of(layers.begin(), layers.end(), alike)) layers.push_back(L);
+  }
   size_t best = 0;
-  for (int n = 16;; n = std::min(n + 16, nmax)) {
-    for (int L = 0; L < m.n_layers; L++) {
+  for (int n = 1;; n = std::min(n < GEMM_QUAD_MAX ? n + 1 : n + 16, nmax)) {
+    for (int L : layers) {
       const gq_weight *qkv[3] = {m.wq[L], m.wk[L], m.wv[L]};
       for (int set = 1; set < 8; set++) {  // whichever of them share a type and so a launch
         const gq_weight *grp[3];

@@ -46,6 +46,27 @@ Q6_TIMES = [
 ]
 
 
+# bf16 calls on the short-batch kernel: (dtype, rows, k, tokens, us unsplit, us in
+# 2 K splits).
+Q8_0 = 8
+SPLIT_TIMES = [
+    (Q4_K, 3584, 1280, 128, 23.9, 20.5), (Q4_K, 4800, 1280, 96, 20.6, 18.7), (Q8_0, 3584, 2048, 128, 22.6, 19.0),
+    (Q8_0, 4800, 2048, 96, 19.9, 17.6), (Q8_0, 9000, 2048, 48, 16.6, 15.5), (Q4_K, 14336, 2048, 48, 16.4, 17.3),
+    (Q8_0, 14336, 2048, 96, 22.3, 24.1), (Q8_0, 14336, 2048, 128, 25.8, 28.1), (Q8_0, 14336, 1280, 128, 23.9, 26.4),
+    (Q6_K, 37888, 3584, 48, 55.9, 58.7), (Q4_K, 37888, 3584, 96, 69.2, 72.4), (Q8_0, 65536, 3584, 64, 99.5, 107.8),
+    (Q4_K, 14336, 2048, 96, 21.0, 24.0), (Q4_K, 14336, 2048, 128, 24.8, 28.5), (Q6_K, 65536, 3584, 128, 132.6, 147.2),
+    (Q8_0, 65536, 3584, 128, 138.0, 149.4), (Q6_K, 37888, 4096, 64, 63.7, 68.2), (Q4_K, 37888, 4096, 128, 82.6, 86.1),
+]
+
+
+def test_quad_split_rule(ask):
+    """A K split earns its reduction, its launch and the partial products'
+    traffic that grows with tokens and rows, to within the estimate's error."""
+    got = ask([f"quad {t} {r} {units(k)} {n}" for t, r, k, n, _, _ in SPLIT_TIMES])
+    for (t, r, k, n, one, two), (ks,) in zip(SPLIT_TIMES, got):
+        assert {1: one, 2: two}[ks] <= 1.1 * min(one, two), f"dtype {t}, {r} x {k} at {n} tokens: {ks} splits"
+
+
 def test_q6_small_rule(ask):
     """The rule takes the faster of the two kernels wherever they differ by
     more than the estimates can tell."""
