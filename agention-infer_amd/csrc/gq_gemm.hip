@@ -585,32 +585,14 @@ hipError_t launch_gemm_records(const gq_weight *w, uint8_t *out, hipStream_t st)
   return hipGetLastError();
 }
 
-int gemm_ksplit(int tiles, int stages, int num_cus) {
-  // The split with the least time per unit of work, rounds / ks (a block
-  // per CU per round; 45 tiles x 6 = 270 blocks would run a second round
-  // of 14), the smaller on ties; at most 8, at least 4 stages per split.
-  if (tiles >= num_cus) return 1;
-  const int kmax = std::max(1, std::min(8, stages / 4));
-  int best = 1;
-  double best_t = 1.0;
-  for (int ks = 2; ks <= kmax; ks++) {
-    const double t = (double)((tiles * ks + num_cus - 1) / num_cus) / ks;
-    if (t < best_t - 1e-9) {
-      best_t = t;
-      best = ks;
-    }
-  }
-  return best;
-}
-
 namespace {
 struct GemmPlan {
   bool quad;                        // gq_gemm_quad.hip's kernel
   int tbm, tbn, ntiles, tiles, ksplit;
 };
-GemmPlan gemm_plan(const gq_weight *const *ws, int count, int n, int num_cus) {
+GemmPlan gemm_plan(const gq_weight *const *ws, int count, int n, bool quad, int num_cus) {
   GemmPlan p;
-  p.quad = gemm_uses_quad(ws, count, n);
+  p.quad = quad;
   p.tbm = p.quad ? GEMM_QUAD_ROWS : BM;
   p.tbn = p.quad ? 16 * gemm_quad_nt(n) : BN;
   p.ntiles = (n + p.tbn - 1) / p.tbn;
@@ -628,15 +610,12 @@ GemmPlan gemm_plan(const gq_weight *const *ws, int count, int n, int num_cus) {
 }
 }  // namespace
 
-// Batches of up to 128 tokens (the largest whose accumulators and X fragments
-// fit a wave's registers), on weights in the quad layout (all dense ones; not
-// stacked experts of other than 16 m rows).  Measured at 128 tokens against
-// the 160 x 256 kernel at 160 (one token tile either way), us a call: 3584 x
-// 18944 Q6_K 47 against 70, 18944 x 3584 Q4_K 44 against 51.
-bool gemm_uses_quad(const gq_weight *const *ws, int count, int n) {
-  for (int i = 0; i < count; i++)
-    if (!ws[i]->L.quad) return false;
-  return n <= GEMM_QUAD_MAX;
+// The short-batch kernel takes up to 128 tokens (the largest batch whose
+// accumulators and X fragments fit a wave's registers), on weights in the quad
+// layout (all dense ones; not stacked experts of other than 16 m rows), where
+// it is the faster one.
+bool gemm_uses_quad(const gq_weight *w, int n, int num_cus) {
+  return w->L.quad && n <= GEMM_QUAD_MAX && gemm_quad_faster(w->L.dtype, w->L.rows, w->L.units, n, num_cus);
 }
 
 // bf16 of X in fragment form for a batch of n (quad: gemm_uses_quad).
@@ -658,20 +637,24 @@ hipError_t launch_reduce(ReduceSegs &r, int ksplit, bool add, hipStream_t st) {
 }
 }  // namespace
 
-size_t gemm_part_floats(const gq_weight *const *ws, int count, int n, int num_cus, bool add) {
-  const GemmPlan p = gemm_plan(ws, count, n, num_cus);
+size_t gemm_part_floats(const gq_weight *const *ws, int count, int n, bool quad, int num_cus, bool add) {
+  const GemmPlan p = gemm_plan(ws, count, n, quad, num_cus);
   if (p.ksplit == 1 && !add) return 0;
   size_t rows = 0;
   for (int i = 0; i < count; i++) rows += (size_t)ws[i]->L.rows;
   return (size_t)p.ksplit * n * rows;
 }
 
+static size_t gemm_bf16_bytes(const gq_weight *w, int n, bool quad, int num_cus) {
+  const size_t xb = gemm_x_elems(w->L.units, n, quad) * 2;
+  return ((xb + 255) & ~(size_t)255) + gemm_part_floats(&w, 1, n, quad, num_cus, false) * 4 + 256;
+}
+
 size_t gemm_workspace_bytes(const gq_weight *w, int n, int mode, int num_cus) {
   if (mode == GQ_GEMM_BF16) {
     if (w->L.dtype != T_Q4_K && w->L.dtype != T_Q6_K && w->L.dtype != T_Q5_K && w->L.dtype != T_Q8_0)
       return (size_t)-1;
-    const size_t xb = gemm_x_elems(w->L.units, n, gemm_uses_quad(&w, 1, n)) * 2;
-    return ((xb + 255) & ~(size_t)255) + gemm_part_floats(&w, 1, n, num_cus, false) * 4 + 256;
+    return gemm_bf16_bytes(w, n, gemm_uses_quad(w, n, num_cus), num_cus);
   }
   if (w->L.dtype != T_Q4_K && w->L.dtype != T_Q6_K) return (size_t)-1;
   return gemm_q8_workspace_bytes(w->L, n, num_cus);
@@ -690,10 +673,10 @@ size_t gemm_workspace_bound(const gq_weight *w, int n, int num_cus) {
   if (nr > 0x7fffff00) return 0;
   const int nmax = (int)nr;
   size_t b = 0;
-  for (int t = 1; t <= GEMM_QUAD_MAX; t++)  // (a split per batch)
-    b = std::max(b, gemm_workspace_bytes(w, t, GQ_GEMM_BF16, num_cus));
-  for (int t = GEMM_NPAD; t <= nmax; t += GEMM_NPAD)
-    b = std::max(b, gemm_workspace_bytes(w, t, GQ_GEMM_BF16, num_cus));
+  for (int t = 1; w->L.quad && t <= GEMM_QUAD_MAX; t++)  // (a split per batch)
+    b = std::max(b, gemm_bf16_bytes(w, t, true, num_cus));
+  for (int t = GEMM_NPAD; t <= nmax; t += GEMM_NPAD)  // (a split per token tile)
+    b = std::max(b, gemm_bf16_bytes(w, t, false, num_cus));
   if (nmax < 512) b = std::max(b, gemm_x_elems(w->L.units, 512, false) * 2 + 256);
   if (w->L.dtype == T_Q4_K || w->L.dtype == T_Q6_K)
     b = std::max(b, q8_bytes_bound(w->L.rows, w->L.units, nmax, num_cus));
@@ -712,11 +695,11 @@ hipError_t launch_x_to_frag(const float *X, int n, int k, uint16_t *xb, hipStrea
 }
 
 hipError_t launch_gemm_bf16(const gq_weight *const *ws, float *const *ys, int count,
-                            const uint16_t *xb, int n, float *part, bool add, int num_cus,
+                            const uint16_t *xb, int n, bool quad, float *part, bool add, int num_cus,
                             hipStream_t st, int *defer) {
-  if (count < 1 || count > GEMM_MAX_SEG || n <= 0) return hipErrorInvalidValue;
+  if (count < 1 || count > GEMM_MAX_SEG || n <= 0 || (quad && n > GEMM_QUAD_MAX)) return hipErrorInvalidValue;
   const int fmt = ws[0]->L.dtype;
-  const GemmPlan p = gemm_plan(ws, count, n, num_cus);
+  const GemmPlan p = gemm_plan(ws, count, n, quad, num_cus);
   const bool parts = add || p.ksplit > 1;  // partial products, summed by k_gemm_reduce
   GemmArgs a{};
   a.nseg = count;
@@ -727,7 +710,7 @@ hipError_t launch_gemm_bf16(const gq_weight *const *ws, float *const *ys, int co
   int tb = 0;
   size_t po = 0;
   for (int i = 0; i < count; i++) {
-    if (ws[i]->L.dtype != fmt || ws[i]->L.units != ws[0]->L.units || !(p.quad || ws[i]->gemm_raw))
+    if (ws[i]->L.dtype != fmt || ws[i]->L.units != ws[0]->L.units || !(quad ? ws[i]->L.quad != 0 : ws[i]->gemm_raw != nullptr))
       return hipErrorInvalidValue;
     a.seg[i].rec = ws[i]->gemm_raw;
     a.seg[i].body = ws[i]->body;
@@ -823,12 +806,12 @@ hipError_t launch_gemm(const gq_weight *w, const float *X, int n, float *Y, int 
   const Layout &L = w->L;
   if (mode == GQ_GEMM_BF16) {
     uint16_t *xb = (uint16_t *)workspace;
-    const bool quad = gemm_uses_quad(&w, 1, n);
+    const bool quad = gemm_uses_quad(w, n, num_cus);
     const size_t xbb = gemm_x_elems(L.units, n, quad) * 2;
     float *part = (float *)((char *)workspace + ((xbb + 255) & ~(size_t)255));
     hipError_t e = quad ? launch_x_to_quad(X, n, L.k, xb, st) : launch_x_to_frag(X, n, L.k, xb, st);
     if (e != hipSuccess) return e;
-    return launch_gemm_bf16(&w, &Y, 1, xb, n, part, false, num_cus, st);
+    return launch_gemm_bf16(&w, &Y, 1, xb, n, quad, part, false, num_cus, st);
   }
   return launch_gemm_q8(w, X, n, Y, workspace, num_cus, st);
 }

@@ -91,6 +91,52 @@ inline int gemm_quad_ksplit(int dtype, int tiles, long rows, int units, int n, i
   return best;
 }
 
+// The 160 x 256 kernel's K split of a launch with this many row x token tiles and
+// 64-element stages.
+inline int gemm_ksplit(int tiles, int stages, int num_cus) {
+  // The split with the least time per unit of work, rounds / ks (a block
+  // per CU per round; 45 tiles x 6 = 270 blocks would run a second round
+  // of 14), the smaller on ties; at most 8, at least 4 stages per split.
+  if (tiles >= num_cus) return 1;
+  const int kmax = std::max(1, std::min(8, stages / 4));
+  int best = 1;
+  double best_t = 1.0;
+  for (int ks = 2; ks <= kmax; ks++) {
+    const double t = (double)((tiles * ks + num_cus - 1) / num_cus) / ks;
+    if (t < best_t - 1e-9) {
+      best_t = t;
+      best = ks;
+    }
+  }
+  return best;
+}
+
+// Its estimated time at up to 256 tokens, us (error 5%): its stages take the same
+// however few the tokens.  A ragged last tile waits on its one last row.
+inline double gemm_direct_time(int dtype, int rows, int units, int n, int num_cus) {
+  const int tiles = (rows + 159) / 160, ks = gemm_ksplit(tiles, 4 * units, num_cus);
+  const double stage = dtype == 12 ? 1.13 : dtype == 13 ? 1.5 : dtype == 14 ? 1.36 : 1.15;
+  const double out = (double)rows * n * 8e-6 / 4.5;
+  const long rounds = ((long)tiles * ks + num_cus - 1) / num_cus;
+  return 3.1 + rounds * (3.4 + stage * ((4 * units + ks - 1) / ks)) + (ks > 1 ? 3.2 + 0.78 * ks * out : 0.0) +
+         0.22 * out + 2.4 * n / 128 + 1.6 * (tiles * 160 - rows) / 160;
+}
+
+// Whether a batch of n <= 128 tokens is faster on the short-batch kernel.  It is,
+// up to four times, but where a row is one unit, and three quarters of the MFMA
+// depth its zeros, or where its lower tiles take one round of blocks more; then
+// the estimates decide.  Measured short / 160 x 256, us a call: 4800 x 256 Q4_K
+// at 64 tokens 12.3 / 12.5, at 97 15.7 / 12.7; 37888 x 256 Q8_0 (339 and 237
+// tiles) at 1 token 14.4 / 12.0, at 128 27.7 / 15.1; 37888 x 512 Q6_K at 32 18.8 /
+// 18.8, at 128 32.1 / 21.5; 18944 x 512 Q4_K at 128 17.9 / 26.2.
+inline bool gemm_quad_faster(int dtype, int rows, int units, int n, int num_cus) {
+  const int tiles = (rows + GEMM_QUAD_ROWS - 1) / GEMM_QUAD_ROWS;
+  const int rounds = (tiles + num_cus - 1) / num_cus, direct = ((rows + 159) / 160 + num_cus - 1) / num_cus;
+  if (units > 1 && rounds <= direct) return true;
+  const int ks = gemm_quad_ksplit(dtype, tiles, rows, units, n, num_cus);
+  return gemm_quad_time(dtype, tiles, rows, units, n, ks, num_cus) <= gemm_direct_time(dtype, rows, units, n, num_cus);
+}
+
 // ----------------------------------------------------------- int8 mode
 // (gq_gemm_q8.hip.)  small: 64 x 64 blocks, no K split; else 160 rows x 128 nj
 // tokens.

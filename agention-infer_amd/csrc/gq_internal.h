@@ -254,25 +254,23 @@ struct GemmArgs {
   int pair, hkpad;
   uint16_t *hb;
 };
-// Batches of up to GEMM_QUAD_MAX tokens run on the quad-layout weights
-// (gq_gemm_quad.hip), whose X fragments cover 16 * gemm_quad_nt(n) tokens;
-// for longer ones X fragments must cover n rounded up to GEMM_NPAD (the
-// 256-token tile).
+// The short-batch kernel (quad: n <= GEMM_QUAD_MAX, weights in the quad layout;
+// gq_gemm_quad.hip) takes X fragments of 16 * gemm_quad_nt(n) tokens, the 160 x
+// 256 kernel of n rounded up to GEMM_NPAD (its token tile).
 constexpr int GEMM_NPAD = 256;
-bool gemm_uses_quad(const gq_weight *const *ws, int count, int n);
+bool gemm_uses_quad(const gq_weight *w, int n, int num_cus);  // gq_gemm's choice
 size_t gemm_x_elems(int units, int n, bool quad);
 hipError_t launch_x_to_quad(const float *X, int n, int k, uint16_t *xb, hipStream_t st);
 hipError_t launch_gemm_quad(const GemmArgs &a, int fmt, int blocks, hipStream_t st);
-// K split of a launch with this many row x token tiles and stages.
-int gemm_ksplit(int tiles, int stages, int num_cus);
 // Y_i (+)= W_i . X for count <= GEMM_MAX_SEG weights of one dtype and in_dim,
-// on X already in fragment form (xb, n tokens; the form gemm_uses_quad tells).
+// on X already in fragment form (xb, n tokens, the form of the kernel that quad
+// tells).
 // add: Y_i += (else =; an accumulating launch writes partials and adds in the
 // reduction).  part: gemm_part_floats floats.
 // defer (accumulating launches only): the reduction is left to the
 // caller; *defer receives the K split whose partials part holds.
 hipError_t launch_gemm_bf16(const gq_weight *const *ws, float *const *ys, int count,
-                            const uint16_t *xb, int n, float *part, bool add, int num_cus,
+                            const uint16_t *xb, int n, bool quad, float *part, bool add, int num_cus,
                             hipStream_t st, int *defer = nullptr);
 // The gate/up pair of the SwiGLU on the direct kernel: hb = bf16 fragments
 // of silu(gate . X) * (up . X) ([npad/16][round_up(F, 256)/32][64][8], the
@@ -281,7 +279,7 @@ hipError_t launch_gemm_bf16(const gq_weight *const *ws, float *const *ys, int co
 // caller then runs launch_gemm_bf16 and its own SwiGLU.
 hipError_t launch_gemm_bf16_swiglu(const gq_weight *gate, const gq_weight *up, const uint16_t *xb, int n,
                                    uint16_t *hb, int num_cus, hipStream_t st);
-size_t gemm_part_floats(const gq_weight *const *ws, int count, int n, int num_cus, bool add);
+size_t gemm_part_floats(const gq_weight *const *ws, int count, int n, bool quad, int num_cus, bool add);
 // X fp32 [n][k] -> bf16 fragments (kpad = k rounded up to 256, npad = n
 // rounded up to GEMM_NPAD, zero padding).
 hipError_t launch_x_to_frag(const float *X, int n, int k, uint16_t *xb, hipStream_t st);

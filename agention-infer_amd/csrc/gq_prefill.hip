@@ -601,6 +601,7 @@ size_t prefill_part_floats(const DecodeLaunch &m, int nmax, int num_cus) {
   }
   size_t best = 0;
   for (int n = 1;; n = std::min(n < GEMM_QUAD_MAX ? n + 1 : n + 16, nmax)) {
+    const bool quad = n <= GEMM_QUAD_MAX;
     for (int L : layers) {
       const gq_weight *qkv[3] = {m.wq[L], m.wk[L], m.wv[L]};
       for (int set = 1; set < 8; set++) {  // whichever of them share a type and so a launch
@@ -608,12 +609,12 @@ size_t prefill_part_floats(const DecodeLaunch &m, int nmax, int num_cus) {
         int c = 0;
         for (int i = 0; i < 3; i++)
           if (set >> i & 1) grp[c++] = qkv[i];
-        best = std::max(best, gemm_part_floats(grp, c, n, num_cus, false));
+        best = std::max(best, gemm_part_floats(grp, c, n, quad, num_cus, false));
       }
-      best = std::max(best, gemm_part_floats(&m.wo[L], 1, n, num_cus, true));
+      best = std::max(best, gemm_part_floats(&m.wo[L], 1, n, quad, num_cus, true));
       const gq_weight *gu[2] = {m.wgate[L], m.wup[L]};
-      best = std::max(best, gemm_part_floats(gu, 2, n, num_cus, false));
-      best = std::max(best, gemm_part_floats(&m.wdown[L], 1, n, num_cus, true));
+      best = std::max(best, gemm_part_floats(gu, 2, n, quad, num_cus, false));
+      best = std::max(best, gemm_part_floats(&m.wdown[L], 1, n, quad, num_cus, true));
     }
     if (n >= nmax) return best;
   }
@@ -650,7 +651,7 @@ hipError_t launch_prefill(const DecodeLaunch &m, const PrefillBufs &b, const int
           gout[c++] = outs[j];
           done[j] = true;
         }
-      if ((e = launch_gemm_bf16(grp, gout, c, b.xb, n, b.part, false, num_cus, s)) != hipSuccess) return e;
+      if ((e = launch_gemm_bf16(grp, gout, c, b.xb, n, quad, b.part, false, num_cus, s)) != hipSuccess) return e;
     }
     uint16_t *kc, *vc;  // the f16 K/V rows the attention reads
     if (m.kv_q8) {
@@ -681,7 +682,7 @@ hipError_t launch_prefill(const DecodeLaunch &m, const PrefillBufs &b, const int
       hipLaunchKernelGGL(k_attn_prefill<64>, ag, dim3(512), 0, s, b.q, kc, vc, pos0, n, nh, group,
                          round_up(qd, kq), quad, b.xb);
     float *xo[1] = {b.x};
-    if ((e = launch_gemm_bf16(&m.wo[L], xo, 1, b.xb, n, b.part, true, num_cus, s, &pending)) != hipSuccess)
+    if ((e = launch_gemm_bf16(&m.wo[L], xo, 1, b.xb, n, quad, b.part, true, num_cus, s, &pending)) != hipSuccess)
       return e;
     hipLaunchKernelGGL(k_norm_to_frag, dim3(npad), dim3(256), 0, s, b.x, m.ffn_norm[L], n, H,
                        round_up(H, kq), quad, m.eps, b.xb, b.part, pending);
@@ -695,7 +696,7 @@ hipError_t launch_prefill(const DecodeLaunch &m, const PrefillBufs &b, const int
     if (e == hipErrorNotSupported) {
       const gq_weight *gu[2] = {m.wgate[L], m.wup[L]};
       float *guo[2] = {b.g, b.u};
-      if ((e = launch_gemm_bf16(gu, guo, 2, b.xb, n, b.part, false, num_cus, s)) != hipSuccess) return e;
+      if ((e = launch_gemm_bf16(gu, guo, 2, b.xb, n, quad, b.part, false, num_cus, s)) != hipSuccess) return e;
       const int kpf = round_up(F, kq);
       hipLaunchKernelGGL(k_swiglu_to_frag, dim3((int)(((long)npad / 16 * (kpf / 32) + 3) / 4)), dim3(256), 0,
                          s, b.g, b.u, n, F, npad, kpf, quad, b.xb);
@@ -704,7 +705,7 @@ hipError_t launch_prefill(const DecodeLaunch &m, const PrefillBufs &b, const int
       return e;
     }
     // (the next layer's norm does the reduction; the head reads x itself)
-    if ((e = launch_gemm_bf16(&m.wdown[L], xo, 1, hx, n, b.part, true, num_cus, s,
+    if ((e = launch_gemm_bf16(&m.wdown[L], xo, 1, hx, n, quad, b.part, true, num_cus, s,
                               L + 1 < m.n_layers ? &pending : nullptr)) != hipSuccess)
       return e;
   }

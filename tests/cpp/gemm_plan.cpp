@@ -1,7 +1,8 @@
 // Answers questions about the batched product's launch rules, one a line, for
 // 256 CUs:
 //   q8 DTYPE ROWS UNITS N               ->  small nj ksplit bytes bound-of-N
-//   quad DTYPE ROWS UNITS N             ->  ksplit of the short-batch bf16 kernel
+//   quad DTYPE ROWS UNITS N             ->  ksplit of the short-batch bf16 kernel,
+//                                           and whether a batch takes that kernel
 //   room N                              ->  tokens that workspace is taken for
 //   take HELD DENIED NEED ROOM LIMIT    ->  ok held denied allocations, where at
 //                                           most LIMIT bytes are to be had
@@ -20,7 +21,8 @@ int main() {
                   gq::q8_bytes_bound(rows, units, n, 256));
     } else if (!std::strcmp(what, "quad") && std::scanf("%d %d %d %d", &dtype, &rows, &units, &n) == 4) {
       const int tiles = (rows + gq::GEMM_QUAD_ROWS - 1) / gq::GEMM_QUAD_ROWS;
-      std::printf("%d\n", gq::gemm_quad_ksplit(dtype, tiles, rows, units, n, 256));
+      std::printf("%d %d\n", gq::gemm_quad_ksplit(dtype, tiles, rows, units, n, 256),
+                  gq::gemm_quad_faster(dtype, rows, units, n, 256));
     } else if (!std::strcmp(what, "room") && std::scanf("%d", &n) == 1) {
       std::printf("%ld\n", gq::gemm_room_tokens(n));
     } else if (!std::strcmp(what, "take")) {

@@ -1,6 +1,15 @@
-"""Shapes of the int8 mode's GPU tests, with the kernel each is there for
-(on 256 CUs): "small" (64 x 64 blocks) or 160 rows x 128 / 256 tokens."""
-Q4_K, Q6_K = 12, 14
+"""Shapes of the batched product's GPU tests that are there for one kernel, on
+256 CUs."""
+Q8_0, Q4_K, Q5_K, Q6_K = 8, 12, 13, 14
+
+# Batches of up to 128 tokens on the 160 x 256 bf16 kernel: one unit a row, one
+# and several row tiles with and without a ragged last one, ragged units.
+BF16_SHORT_DIRECT = [
+    (Q4_K, 480, 256, 97), (Q5_K, 4785, 256, 128), (Q6_K, 14335, 256, 113), (Q8_0, 4800, 224, 128),
+    (Q4_K, 37888, 131, 33), (Q8_0, 37889, 512, 128),
+]
+
+# The int8 mode: "small" (64 x 64 blocks) or 160 rows x 128 / 256 tokens.
 
 # (dtype, rows, k, n, kernel)
 INT8_KERNELS = [

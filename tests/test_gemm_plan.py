@@ -4,7 +4,7 @@ import subprocess
 
 import pytest
 
-from gemm_shapes import INT8_KERNELS, Q4_K, Q6_K
+from gemm_shapes import BF16_SHORT_DIRECT, INT8_KERNELS, Q4_K, Q5_K, Q6_K, Q8_0
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 
@@ -31,6 +31,26 @@ def units(k):
     return (k + 255) // 256
 
 
+# bf16 calls: (dtype, rows, k, tokens, us on the short-batch kernel, us on the
+# 160 x 256 one).
+SHORT_TIMES = [
+    (Q4_K, 4800, 256, 64, 12.3, 12.5), (Q4_K, 4800, 256, 97, 15.7, 12.7), (Q4_K, 9000, 256, 64, 12.4, 14.9),
+    (Q6_K, 18944, 256, 128, 18.1, 15.6), (Q8_0, 9000, 256, 64, 11.5, 14.7), (Q5_K, 14336, 256, 128, 17.7, 15.5),
+    (Q6_K, 1200, 256, 16, 11.6, 12.9), (Q6_K, 4800, 512, 128, 16.8, 18.6), (Q4_K, 18944, 512, 128, 17.9, 26.2),
+    (Q4_K, 18944, 3584, 64, 29.8, 45.9), (Q4_K, 37888, 256, 32, 14.4, 12.7), (Q8_0, 37888, 256, 1, 14.4, 12.0),
+    (Q8_0, 37888, 256, 128, 27.7, 15.1), (Q6_K, 37888, 512, 128, 32.1, 21.5), (Q4_K, 37888, 1024, 128, 32.1, 28.7),
+    (Q6_K, 65536, 256, 64, 31.1, 25.1), (Q8_0, 65536, 512, 112, 41.6, 33.7), (Q8_0, 128256, 256, 96, 54.4, 42.9),
+]
+
+
+def test_quad_kernel_rule(ask):
+    """A short batch takes the faster kernel, to within the estimates' error."""
+    got = ask([f"quad {t} {r} {units(k)} {n}" for t, r, k, n, _, _ in SHORT_TIMES])
+    for (t, r, k, n, short, direct), (_, quad) in zip(SHORT_TIMES, got):
+        taken, other = (short, direct) if quad else (direct, short)
+        assert taken <= 1.1 * other, f"dtype {t}, {r} x {k} at {n} tokens: takes {taken} us, the other {other}"
+
+
 # Q6_K int8 calls: (rows, k, tokens, us on the 64 x 64 blocks, us on the
 # 160-row ones with their K split).
 Q6_TIMES = [
@@ -48,7 +68,6 @@ Q6_TIMES = [
 
 # bf16 calls on the short-batch kernel: (dtype, rows, k, tokens, us unsplit, us in
 # 2 K splits).
-Q8_0 = 8
 SPLIT_TIMES = [
     (Q4_K, 3584, 1280, 128, 23.9, 20.5), (Q4_K, 4800, 1280, 96, 20.6, 18.7), (Q8_0, 3584, 2048, 128, 22.6, 19.0),
     (Q8_0, 4800, 2048, 96, 19.9, 17.6), (Q8_0, 9000, 2048, 48, 16.6, 15.5), (Q4_K, 14336, 2048, 48, 16.4, 17.3),
@@ -63,7 +82,7 @@ def test_quad_split_rule(ask):
     """A K split earns its reduction, its launch and the partial products'
     traffic that grows with tokens and rows, to within the estimate's error."""
     got = ask([f"quad {t} {r} {units(k)} {n}" for t, r, k, n, _, _ in SPLIT_TIMES])
-    for (t, r, k, n, one, two), (ks,) in zip(SPLIT_TIMES, got):
+    for (t, r, k, n, one, two), (ks,) in zip(SPLIT_TIMES, ((g[0],) for g in got)):
         assert {1: one, 2: two}[ks] <= 1.1 * min(one, two), f"dtype {t}, {r} x {k} at {n} tokens: {ks} splits"
 
 
@@ -76,7 +95,9 @@ def test_q6_small_rule(ask):
         assert taken <= 1.05 * other, f"{r} x {k} at {n} tokens: takes {taken} us, the other {other}"
 
 
-def test_int8_test_shapes_take_their_kernel(ask):
+def test_test_shapes_take_their_kernel(ask):
+    got = ask([f"quad {t} {r} {units(k)} {n}" for t, r, k, n in BF16_SHORT_DIRECT])
+    assert [g[1] for g in got] == [0] * len(got)
     got = ask([f"q8 {t} {r} {units(k)} {n}" for t, r, k, n, _ in INT8_KERNELS])
     for (t, r, k, n, kernel), g in zip(INT8_KERNELS, got):
         assert kernel == ("small" if g[0] else 128 * g[1]), f"dtype {t}, {r} x {k} at {n} tokens: {g}"

@@ -17,7 +17,7 @@ import numpy as np
 import pytest
 
 import gq_synth as syn
-from gemm_shapes import INT8_KERNELS
+from gemm_shapes import BF16_SHORT_DIRECT, INT8_KERNELS
 
 pytestmark = pytest.mark.gpu
 
@@ -91,6 +91,16 @@ def test_gemm_bf16_short(backend, orc, dtype, rows, k, n):
     112 with remainders, last quads of 1 to 4 units, K split or not."""
     import gq
     say(f"gemm bf16 short dtype={dtype} rows={rows} k={k} n={n}")
+    w, X, Wf, Y = run(backend, orc, rows, k, n, gq.GQ_GEMM_BF16, seed=rows + 3 * k + n, dtype=dtype)
+    ref = bf16_round(X).astype(np.float64) @ bf16_round(Wf).astype(np.float64).T
+    check(Y, ref, "bf16 vs same-operand fp64")
+
+
+@pytest.mark.parametrize("dtype,rows,k,n", BF16_SHORT_DIRECT)
+def test_gemm_bf16_short_direct(backend, orc, dtype, rows, k, n):
+    """Batches of up to 128 tokens that take the 160 x 256 kernel."""
+    import gq
+    say(f"gemm bf16 short direct dtype={dtype} rows={rows} k={k} n={n}")
     w, X, Wf, Y = run(backend, orc, rows, k, n, gq.GQ_GEMM_BF16, seed=rows + 3 * k + n, dtype=dtype)
     ref = bf16_round(X).astype(np.float64) @ bf16_round(Wf).astype(np.float64).T
     check(Y, ref, "bf16 vs same-operand fp64")
