@@ -99,9 +99,11 @@ __global__ __launch_bounds__(256) void k_x_to_q8(const float *X, int n, int npad
                (_Float16)(float)q[4], (_Float16)(float)q[6], (_Float16)(float)q[5], (_Float16)(float)q[7]};
   *(h16x8_t *)(xq + (f * 64 + lane) * 8) = o;
   if (xm) {
-    const float x = sc * (float)sum, x1 = __uint_as_float(f2bf(x) << 16), x2 = __uint_as_float(f2bf(x - x1) << 16);
+    const float x = sc * (float)sum, x1 = __uint_as_float(f2bf(x) << 16);
+    // (past the f16 scale's range x is infinite, or 0 inf, and all of it is in x1)
+    const float rest = fabsf(x) < INFINITY ? x - x1 : 0.f, x2 = __uint_as_float(f2bf(rest) << 16);
     xm[(((long)nt * units + (kb >> 3)) * 64 + lane) * 8 + (kb & 7)] =
-        (uint16_t)f2bf(sub == 0 ? x1 : sub == 1 ? x2 : sub == 2 ? (x - x1) - x2 : 0.f);
+        (uint16_t)f2bf(sub == 0 ? x1 : sub == 1 ? x2 : sub == 2 ? rest - x2 : 0.f);
   }
 }
 

@@ -206,6 +206,34 @@ def test_gemm_int8_kernels(backend, orc, dtype, rows, k, n, kernel):
         assert err.max() <= (1e-6 if rows > 1 else 1e-5)
 
 
+@pytest.mark.parametrize("dtype", [Q4_K, Q6_K])
+def test_gemm_int8_scale_overflow(backend, orc, dtype):
+    """A block whose f16 scale overflows gives infinite products: results of
+    one sign stay infinite, and other tokens finite.  (Q4_K with a negative
+    dmin, so that the min term has the dot's sign.)"""
+    import gq
+    import torch
+    rows, k, n = 37, 512, 5
+    w = syn.make_blocks(dtype, rows, k, seed=81)
+    if dtype == Q4_K:
+        b = w.reshape(rows, -1, 144)
+        b[..., 0:4] = np.array([0.01, -0.01], np.float16).view(np.uint8)
+        b[..., 4:16] = 0x21  # scales and mins 33 or more than 0
+    else:
+        b = w.reshape(rows, -1, 210)
+        b[..., 128:192] |= 0xAA  # codes above 32
+        b[..., 0:128] |= 0x11
+        b[..., 192:208] = 5
+    X = syn.make_x(k, seed=82, batch=n)
+    X[1, 64:96] = 1e7
+    X[3, 256:288] = -1e7
+    h = backend.upload_weight(dtype, w, k, rows)
+    Y = h.launch_only_batch(torch.from_numpy(X).cuda(), mode=gq.GQ_GEMM_INT8).cpu().numpy()
+    assert np.all(Y[1] == np.inf) and np.all(Y[3] == -np.inf)
+    fin = [0, 2, 4]
+    check(Y[fin], int8_ref(orc, dtype, w, X[fin]), "other tokens")
+
+
 def test_gemm_full_config(backend, orc):
     """config 2: Q4_K 18944 x 3584 times 512 tokens, both modes."""
     import gq
