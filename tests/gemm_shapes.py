@@ -9,12 +9,16 @@ BF16_SHORT_DIRECT = [
     (Q4_K, 37888, 131, 33), (Q8_0, 37889, 512, 128),
 ]
 
-# The int8 mode: "small" (64 x 64 blocks) or 160 rows x 128 / 256 tokens.
-
-# (dtype, rows, k, n, kernel)
+# The int8 mode: (dtype, rows, k, n, kernel), the kernel "small" (64 x 64 blocks)
+# or the tokens of its 160-row blocks.
 INT8_KERNELS = [
     # one unit and several, one block and several, each with a ragged last
     # row tile, token tile and unit
     (Q6_K, 1, 256, 1, "small"), (Q6_K, 63, 130, 64, "small"), (Q6_K, 130, 256, 200, "small"),
     (Q6_K, 65, 512, 65, "small"), (Q6_K, 300, 721, 129, "small"), (Q6_K, 2405, 768, 701, "small"),
+    # one unit (the kernel without a unit's running sum), several, and K splits
+    (Q4_K, 161, 250, 129, 128), (Q4_K, 159, 721, 127, 128), (Q4_K, 161, 1500, 129, 128),
+    (Q6_K, 9001, 250, 509, 128), (Q6_K, 600, 1000, 9, 128), (Q6_K, 161, 1500, 129, 128),
+    (Q4_K, 18945, 250, 257, 256), (Q4_K, 9003, 721, 600, 256), (Q4_K, 2405, 2500, 129, 256),
+    (Q6_K, 18945, 250, 257, 256), (Q6_K, 9003, 721, 600, 256), (Q6_K, 2405, 2500, 129, 256),
 ]

@@ -144,10 +144,12 @@ def test_gemm_int8(backend, orc, dtype, rows, k, n):
 @pytest.mark.parametrize("dtype", [Q4_K, Q6_K])
 @pytest.mark.parametrize("rows,k,n", [(1, 256, 1), (161, 1536, 129), (321, 2560, 257), (2400, 768, 384), (159, 5000, 128)])
 def test_gemm_int8_tiles(backend, orc, dtype, rows, k, n):
-    """Both token tiles (128 and 256), one row past a tile and one short of
-    it, K splits of uneven units, a ragged last unit; Q6_K scales at both
-    ends of int8, where sc (q - 32) passes 11 bits, and activations whose
-    blocks differ by 2^30 in one unit."""
+    """The 128-token tile (both are in test_gemm_int8_kernels), one row past a
+    tile and one short of it, K splits of uneven units, a ragged last unit;
+    Q6_K scales at both ends of int8, where sc (q - 32) passes 11 bits, and
+    activations whose blocks differ by 2^16 in one unit.  In every third token
+    only the small block is left, and errors count against the token's own
+    results (bound: test_gemm_int8_kernels)."""
     import gq
     import torch
     say(f"gemm int8 tiles dtype={dtype} rows={rows} k={k} n={n}")
@@ -157,15 +159,12 @@ def test_gemm_int8_tiles(backend, orc, dtype, rows, k, n):
         b = w.reshape(rows, -1, 210)
         b[..., 192:208] = rng.integers(-128, 128, b[..., 192:208].shape, dtype=np.int8).view(np.uint8)
     X = syn.make_x(k, seed=n, batch=n)
-    X[:, :32] *= np.float32(2.0 ** -30)
+    X[:, :32] *= np.float32(2.0 ** -8)  # (scales of 1e-4 and 5, both normal in f16)
+    X[:, 32:64] *= np.float32(2.0 ** 8)
+    X[::3, 32:] = 0
     h = backend.upload_weight(dtype, w, k, rows)
     Y = h.launch_only_batch(torch.from_numpy(X).cuda(), mode=gq.GQ_GEMM_INT8).cpu().numpy()
-    Wf = orc.dequant_rows(dtype, w, k).astype(np.float64)
-    Xq = np.zeros((n, (k + 31) // 32 * 32), np.float64)
-    for t in range(n):
-        sc, q = orc.quantize_q8_32(X[t])
-        Xq[t, :q.size] = q.astype(np.float64) * np.repeat(sc.view(np.float16).astype(np.float64), 32)[:q.size]
-    check(Y, Xq[:, :k] @ Wf.T, "int8 vs same-operand fp64")
+    check_tokens(Y, int8_ref(orc, dtype, w, X), 1e-6 if rows > 1 else 1e-5)
 
 
 def int8_ref(orc, dtype, w, X):
@@ -178,12 +177,21 @@ def int8_ref(orc, dtype, w, X):
     return Xq @ orc.dequant_rows(dtype, w, k).astype(np.float64).T
 
 
+def check_tokens(Y, ref, tol):
+    """Every token's error against the size of its own results (2-norms)."""
+    assert np.all(np.isfinite(Y))
+    err = np.sqrt(np.mean((Y - ref) ** 2, axis=1)) / np.sqrt(np.mean(ref ** 2, axis=1) + 1e-300)
+    say(f"  worst token {err.max():.3g}, bound {tol:.3g}")
+    assert err.max() <= tol
+
+
 @pytest.mark.parametrize("dtype,rows,k,n,kernel", INT8_KERNELS)
 def test_gemm_int8_kernels(backend, orc, dtype, rows, k, n, kernel):
     """Each kernel of the int8 mode at the edges of its tiles.  Every integer
-    in it is exact, so per token only the roundings of up to 8 units + 2 f32
-    sums and the reference's f32 weights are left: 2^-24 each of terms of the
-    result's size, below 1e-6 of it together."""
+    in it is exact, so per token only the roundings of 8 sums per unit and one
+    or two per unit of the result, and the reference's f32 weights, are left: up
+    to 2^-24 each of partial sums below the result's size, about 1.5e-7 together
+    for 20 units, bounded here by 1e-6."""
     import gq
     import torch
     say(f"gemm int8 {kernel} dtype={dtype} rows={rows} k={k} n={n}")
@@ -194,16 +202,42 @@ def test_gemm_int8_kernels(backend, orc, dtype, rows, k, n, kernel):
         b[..., 192:208] = rng.integers(-128, 128, b[..., 192:208].shape, dtype=np.int8).view(np.uint8)
     X = syn.make_x(k, seed=n, batch=n)
     ref = int8_ref(orc, dtype, w, X)
-    size = np.sqrt(np.mean(ref ** 2, axis=1) + 1e-300)
     h = backend.upload_weight(dtype, w, k, rows)
     for off in (0, 1):  # X aligned, and to 4 bytes only
         buf = torch.zeros(n * k + 1, device="cuda")
         buf[off:off + n * k] = torch.from_numpy(X).cuda().view(-1)
         Y = h.launch_only_batch(buf[off:off + n * k].view(n, k), mode=gq.GQ_GEMM_INT8).cpu().numpy()
-        err = np.sqrt(np.mean((Y - ref) ** 2, axis=1)) / size
-        say(f"  worst token {err.max():.3g}")
-        # (one row: the result may be small beside its terms)
-        assert err.max() <= (1e-6 if rows > 1 else 1e-5)
+        check_tokens(Y, ref, 1e-6 if rows > 1 else 1e-5)  # (one row: it may be small beside its terms)
+
+
+@pytest.mark.parametrize("rows,k,n", [(320, 1024, 130), (18944, 250, 260)])
+def test_gemm_int8_min_term(backend, orc, rows, k, n):
+    """Q4_K results that are all min term: xs sum(q) has 23 bits and goes through
+    the MFMA in three bf16.  What is left is f32 rounding (as in
+    test_gemm_int8_kernels, below 5e-7); a product with two of the three is
+    further off than that."""
+    import gq
+    import torch
+    say(f"gemm int8 min term rows={rows} k={k} n={n}")
+    w = syn.make_blocks(Q4_K, rows, k, seed=91)
+    b = w.reshape(rows, -1, 144)
+    b[..., 0:2] = np.zeros(1, np.float16).view(np.uint8)  # d = 0
+    X = syn.make_x(k, seed=92, batch=n)
+    ref = int8_ref(orc, Q4_K, w, X)
+    xs, m = np.zeros((n, (k + 31) // 32)), np.zeros((rows, (k + 31) // 32))
+    for t in range(n):
+        sc, q = orc.quantize_q8_32(X[t])
+        q = np.pad(q.astype(np.float64), (0, 32 * xs.shape[1] - q.size)).reshape(-1, 32)
+        xs[t] = sc.view(np.float16).astype(np.float64)[:xs.shape[1]] * q.sum(1)
+    m = -orc.dequant_rows(Q4_K, w, k).astype(np.float64)[:, ::32]
+    x1 = bf16_round(xs)
+    two = x1.astype(np.float64) + bf16_round(xs - x1)
+    size = np.sqrt(np.mean(ref ** 2, axis=1))
+    assert np.allclose(-xs @ m.T, ref, rtol=0, atol=1e-9 * np.abs(ref).max())
+    assert (np.sqrt(np.mean(((two - xs) @ m.T) ** 2, axis=1)) / size).max() > 1e-6
+    h = backend.upload_weight(Q4_K, w, k, rows)
+    Y = h.launch_only_batch(torch.from_numpy(X).cuda(), mode=gq.GQ_GEMM_INT8).cpu().numpy()
+    check_tokens(Y, ref, 5e-7)
 
 
 @pytest.mark.parametrize("dtype", [Q4_K, Q6_K])
