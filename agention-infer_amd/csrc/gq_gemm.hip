@@ -524,8 +524,8 @@ __global__ __launch_bounds__(512) void k_gemm_bf16_direct(GemmArgs a) {
       const int t = n0 + 64 * wave + 16 * jn + (lane & 15);
       if (t >= a.n) continue;
       float *yp = Y + (long)t * rows + m;
-      if (m + 3 < rows && (rows & 3) == 0) {
-        *(float4 *)yp = make_float4(acc[i][jn][0], acc[i][jn][1], acc[i][jn][2], acc[i][jn][3]);
+      if (m + 3 < rows) {
+        store4(yp, acc[i][jn]);
       } else {
 #pragma unroll
         for (int r = 0; r < 4; r++)

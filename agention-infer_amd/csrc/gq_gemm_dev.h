@@ -12,6 +12,12 @@ typedef float f32x4_t __attribute__((ext_vector_type(4)));
 typedef int i32x4_t __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(3))) void lds_void_t;
 
+// Four floats to p, aligned to 4 bytes: one store (global memory takes 16 bytes at
+// any dword).  A result row of any other than 4 m rows starts anywhere, and a dword
+// store per element there is four times the requests.
+typedef float f32x4u_t __attribute__((ext_vector_type(4), aligned(4)));
+__device__ __forceinline__ void store4(float *p, f32x4_t v) { *(f32x4u_t *)p = v; }
+
 constexpr int FR16 = 512;  // bf16 per 1 KiB MFMA operand fragment
 
 // fp32 -> bf16 bits, round to nearest even (NaN kept quiet).

@@ -391,8 +391,8 @@ __global__ __launch_bounds__(512) void k_gemm_q8(Q8Args a) {
       const int t = n0 + 16 * (NJ * wave + jn) + (lane & 15);
       if (t >= a.n) continue;
       float *yp = Y + (long)t * rows + m;
-      if (m + 3 < rows && (rows & 3) == 0) {
-        *(float4 *)yp = make_float4(y[i][jn][0], y[i][jn][1], y[i][jn][2], y[i][jn][3]);
+      if (m + 3 < rows) {
+        store4(yp, y[i][jn]);
       } else {
 #pragma unroll
         for (int r = 0; r < 4; r++)

@@ -245,8 +245,8 @@ __global__ __launch_bounds__(64 * (NCW + 1)) void k_gemm_quad(GemmArgs a) {
     const int t = 16 * nt + r;
     if (t >= a.n) continue;
     float *yp = Y + (long)t * rows + m;
-    if (m + 3 < rows && (rows & 3) == 0) {
-      *(float4 *)yp = make_float4(acc[nt][0], acc[nt][1], acc[nt][2], acc[nt][3]);
+    if (m + 3 < rows) {
+      store4(yp, acc[nt]);
     } else {
 #pragma unroll
       for (int i = 0; i < 4; i++)

@@ -268,6 +268,39 @@ def test_gemm_int8_scale_overflow(backend, orc, dtype):
     check(Y[fin], int8_ref(orc, dtype, w, X[fin]), "other tokens")
 
 
+@pytest.mark.parametrize("mode,dtype,rows,k,n", [(0, Q4_K, 10611, 256, 959), (0, Q4_K, 40003, 512, 128),
+                                                 (1, Q6_K, 10611, 512, 959), (1, Q4_K, 3891, 256, 987)])
+def test_gemm_odd_rows(backend, mode, dtype, rows, k, n):
+    """Row counts other than 4 m: results start at any dword, at no cost of a
+    store per element (10611 x 512 Q6_K at 959 tokens: 81 us with that, 59
+    without, 59 for 10612 rows), and the rows past the last are not written."""
+    import torch
+    say(f"gemm odd rows mode={mode} dtype={dtype} rows={rows} k={k} n={n}")
+    w = syn.make_blocks(dtype, rows + 1, k, seed=93)
+    X = torch.from_numpy(syn.make_x(k, seed=94, batch=n)).cuda()
+    us, got = [], []
+    for r in (rows, rows + 1):
+        assert r == rows or r % 4 == 0
+        h = backend.upload_weight(dtype, np.ascontiguousarray(w[:r]), k, r)
+        buf = torch.full((n * r + 9,), 7.0, device="cuda")
+        Y = buf[1:1 + n * r].view(n, r)
+        t = []
+        for i in range(6):
+            a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            a.record()
+            for _ in range(20):
+                h.launch_only_batch(X, mode=mode, Y_dev=Y)
+            b.record()
+            torch.cuda.synchronize()
+            t.append(a.elapsed_time(b) / 20 * 1e3)
+        us.append(min(t))
+        assert buf[0] == 7.0 and torch.all(buf[1 + n * r:] == 7.0)
+        got.append(Y)
+    assert torch.equal(got[0], got[1][:, :rows])
+    say(f"  {us[0]:.1f} us, {us[1]:.1f} for one row more")
+    assert us[0] <= 1.15 * us[1]
+
+
 def test_gemm_full_config(backend, orc):
     """config 2: Q4_K 18944 x 3584 times 512 tokens, both modes."""
     import gq
