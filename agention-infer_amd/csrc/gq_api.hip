@@ -693,7 +693,9 @@ int gq_gemm(const gq_weight *w, const float *X_dev, int n, float *Y_dev, int mod
     return fail(GQ_EDTYPE, "gq_gemm: %s weights not supported in %s mode", type_name(w->L.dtype),
                 mode == GQ_GEMM_BF16 ? "bf16" : "int8");
   {
-    int rc2 = gq_ensure_gemm_records(w, (hipStream_t)stream);  // both modes read the ggml-order copy
+    // Every kernel but the short-batch one reads this copy.  It is made on a
+    // weight's first call of any size, so that one call lets all be captured.
+    int rc2 = gq_ensure_gemm_records(w, (hipStream_t)stream);
     if (rc2) return rc2;
   }
   // An eager call takes room for every call of up to n tokens, so that these

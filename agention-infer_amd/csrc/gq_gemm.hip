@@ -1,5 +1,7 @@
 // gq_gemm.hip -- batched prefill GEMM Y[n][m] = sum_k W[m][k] X[n][k] for
-// Q4_K weights (gfx950 MFMA).
+// Q4_K, Q5_K, Q6_K and Q8_0 weights (gfx950 MFMA): the bf16 kernel for long
+// batches, the K split's reduction, the GEMM copy of a weight, and the choice
+// between the kernels.
 //
 // Replaces the prefill contraction of WeightMap::matmul_batch_into
 // (src/model/mod.rs:414-464: dequant each row once, dot it with every
@@ -17,8 +19,8 @@
 // Tiling (bf16): a block computes 160 weight rows x 256 tokens (18944 rows
 // x 512 tokens -> 238 blocks, one round on 256 CUs).  K advances 64
 // elements (one Q4_K group) per stage, X fragments come straight from L2 into
-// the multiply waves' registers.  Batches of up to 128 tokens take
-// gq_gemm_quad.hip's kernel instead.
+// the multiply waves' registers.  Most batches of up to 128 tokens take
+// gq_gemm_quad.hip's kernel instead (gemm_quad_faster).
 #include <algorithm>
 #include <type_traits>
 

@@ -18,13 +18,17 @@
 // unit: m (6 bits, exact) against xs sum q in three bf16 (24 bits, exact, any
 // exponent), the three at depths 0-7, 8-15 and 16-23.
 // (Activations as f16 pairs hi + lo of xs q, whose dots chain through a whole
-// unit on the MFMAs alone, took 151 us against 130 on 18944 x 3584 x 512, and
-// their longer fp32 chains doubled the error of a short k.)
+// unit on the MFMAs alone, took 151 us of kernel against 130 on 18944 x 3584 x
+// 512, and their longer fp32 chains doubled the error of a short k.)
 //
-// 18944 x 3584 x 512 Q4_K: 130 us of kernel, 204 on int8 MFMA; 3584 x 18944 x 512
-// Q6_K 180 against 450.  The bound is what a SIMD's two waves leave unhidden
-// beside the MFMAs (31 and 62 us at peak rate): the FMAs, staging W, the units'
-// ends, the X loads.
+// 18944 x 3584 x 512 Q4_K: 204 us a call on int8 MFMA, 125 so (kernel 130 to 134
+// under the profiler, which runs one launch at a time); 3584 x 18944 x 512 Q6_K
+// 446 and 183 (kernel 181).  Q4_K / Q6_K, the MFMAs are busy for 25 / 34% of the
+// kernel's cycles (of 93 / 90% of the CUs), VALU issue for 45 / 40%, and on a
+// CU the LDS for 23 / 29%, with waves waiting for it in 2 / 5% of theirs: the
+// bound is what a SIMD's two waves leave unhidden beside the MFMAs, that is the
+// FMAs, staging W, the units' ends and the X loads, and not the A fragments'
+// LDS reads.
 #include <algorithm>
 #include <type_traits>
 
@@ -116,7 +120,6 @@ struct Q8Args {
   int rows, n, kpad, ntiles, ksplit;
 };
 
-
 __device__ __forceinline__ uint32_t pkfma(uint32_t a, h16x2_t s, h16x2_t c) {
   const h16x2_t v = __builtin_bit_cast(h16x2_t, a);
   return __builtin_bit_cast(uint32_t, __builtin_elementwise_fma(v, s, c));
@@ -130,9 +133,10 @@ __device__ __forceinline__ uint32_t pkfma(uint32_t a, h16x2_t s, h16x2_t c) {
 // codes) turn W into f16 fragments in LDS and, on a unit's first stage, write
 // the row's d (and dmin and mins).  One barrier per stage.
 // PROD (k <= 256): y += (d xs) D instead, an instruction more per result and
-// one rounding less, which shows where there is only one unit (Q6_K: 5.3e-8
-// relative error against 5.9e-8; from two units on the other form's is the
-// smaller one).
+// one rounding less, which shows where there is only one unit: relative error
+// 5.4e-8 against 5.9e-8 (Q6_K) and 1.2e-7 against 1.3e-7 (Q4_K), at a price of 8 to
+// 15% (18944 x 256 x 512: 24 against 21.5 us a call, Q6_K 26 against 23.6).  From
+// two units on the other form's error is the smaller one.
 template <int FMT, int NJ, bool PROD>
 __global__ __launch_bounds__(512) void k_gemm_q8(Q8Args a) {
   constexpr bool Q4 = FMT == T_Q4_K;

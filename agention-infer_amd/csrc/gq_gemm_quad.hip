@@ -27,10 +27,11 @@
 // split over quads where the rows alone do not fill the CUs.  One barrier per
 // piece of PS steps.
 //
-// What bounds it now: the dequant's VALU (about 30 instructions per 8 elements
-// and lane, 4 cycles each), 60% busy; the K split leaves the blocks 2 or 3
-// quads each.  3584 x 18944 Q6_K at 37 tokens: 25 us of kernel in a 32 us
-// call, against 63.5 of 70 on 160 x 256 tiles.
+// What bounds it now: latency between the dequant's VALU (about 30 instructions
+// per 8 elements and lane, 4 cycles each; issuing for 36% of the kernel's time on
+// the SIMDs that hold a block) and the MFMAs (13%), with two waves a SIMD; the K
+// split leaves the blocks 2 or 3 quads each.  3584 x 18944 Q6_K at 37 tokens: 70 us
+// a call on 160 x 256 tiles, 31.5 so (kernel 63.5 and 25.8 under the profiler).
 #include <algorithm>
 
 #include "gq_gemm_dev.h"

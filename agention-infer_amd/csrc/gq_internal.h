@@ -223,7 +223,7 @@ hipError_t launch_gemm_q8(const gq_weight *w, const float *X, int n, float *Y, v
                           hipStream_t st);
 // y[i] = sum_s part[s][i], s in order, i < count.
 hipError_t launch_gemm_reduce(const float *part, float *y, long count, int ksplit, hipStream_t st);
-// The bf16 GEMM's per-stage weight records (Q4_K, Q6_K): their size, and
+// The GEMM copy of a dense weight, per-stage records: their size, and
 // their construction from the device's tiled body.
 size_t gemm_records_bytes(const Layout &L);
 hipError_t launch_gemm_records(const gq_weight *w, uint8_t *out, hipStream_t st);

@@ -107,7 +107,8 @@ def cpu_baseline(mats, host, xs, nthreads, budget_s=15.0):
 
 
 DECODE_PREFILL, DECODE_STEPS = 4096, 128
-MFMA_PEAK_TFLOPS = {"bf16": 2500.0, "int8": 5000.0}  # dense, no sparsity
+# Dense, no sparsity.  The int8 mode's integers run as f16 operands.
+MFMA_PEAK_TFLOPS = {"bf16": 2500.0, "int8": 2500.0}
 
 
 def _timed(torch, fn, reps):
@@ -123,7 +124,7 @@ def _timed(torch, fn, reps):
 
 def gemm_leg(be, gq, syn, torch, cpu):
     """Q4_K 18944x3584 weights times 512 tokens of
-    3584 activations, bf16 dequant-to-LDS MFMA and per-32 Q8 int8 MFMA."""
+    3584 activations, bf16 dequant-to-LDS MFMA and per-32 Q8 (exact products on f16 MFMA)."""
     rows, k, n = FFN, HID, 512
     w = syn.make_blocks(Q4_K, rows, k, seed=31)
     h = be.upload_weight(Q4_K, w, k, rows)
