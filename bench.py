@@ -67,7 +67,7 @@ def algo_bytes(gq, dtype, out_dim, in_dim):
 
 
 # Host threads for the CPU legs: every core this process may use, capped at
-# the GPU box's CPU share for one GPU (16 threads).
+# one GPU's share of a host (16 threads).
 BOX_CPU_SHARE = 16
 
 
@@ -123,7 +123,7 @@ def _timed(torch, fn, reps):
 
 
 def gemm_leg(be, gq, syn, torch, cpu):
-    """BASELINE configs[2]: Q4_K 18944x3584 weights times 512 tokens of
+    """Q4_K 18944x3584 weights times 512 tokens of
     3584 activations, bf16 dequant-to-LDS MFMA and per-32 Q8 (exact products on f16 MFMA)."""
     rows, k, n = FFN, HID, 512
     w = syn.make_blocks(Q4_K, rows, k, seed=31)
@@ -171,7 +171,7 @@ def gemm_leg(be, gq, syn, torch, cpu):
 
 
 def q8_0_leg(be, gq, syn, torch, cpu):
-    """BASELINE configs[0]: Q8_0 matvec at the Llama-3.2-1B FFN-up shape,
+    """Q8_0 matvec at the Llama-3.2-1B FFN-up shape,
     W 8192x2048, batch 1.  The matrix is 17.8 MB, so Q8_COPIES device copies
     (356 MB, over the 256 MB Infinity Cache) are cycled to read cold HBM;
     one graph of Q8_COPIES launches, timed with events on its stream."""
@@ -219,7 +219,7 @@ Q8_COPIES = 20
 
 
 def moe_leg(be, gq, syn, torch, cpu):
-    """BASELINE configs[4]: 256 IQ3_XXS experts (gate/up 1536x3072, down
+    """256 IQ3_XXS experts (gate/up 1536x3072, down
     3072x1536), top-8 routing from N(0,1) logits, T = 1, 4, 16 tokens.
     GB/s counts the weight bytes of the distinct experts a call touches."""
     E, H, F, K = 256, 3072, 1536, 8
@@ -327,7 +327,7 @@ def q8_kv_leg(gq, cfg, hw, torch, stream):
 
 
 def decode_leg(be, gq, syn, torch, cpu_steps):
-    """BASELINE configs[3]: GPU-resident 7B-shape Q4_K_M decode (28 layers,
+    """GPU-resident 7B-shape Q4_K_M decode (28 layers,
     f16 KV prefilled to 4096 positions, 128 greedy steps, one HIP graph
     replay per step).  Returns the figures and the oracle's host-side
     decode rate on a bounded sample (cpu_steps steps, same model)."""
@@ -390,7 +390,7 @@ def main():
                     help="run only this leg and print its figures (for profiling)")
     ap.add_argument("--cpu-decode-steps", type=int, default=3)
     ap.add_argument("--decode-steps", type=int, default=DECODE_STEPS,
-                    help="greedy steps timed in the decode legs (128: BASELINE configs[3])")
+                    help="greedy steps timed in the decode legs (default 128)")
     ap.add_argument("--calib-copy", action="store_true",
                     help="also run a plain 256 MiB device copy (HBM counter calibration)")
     args = ap.parse_args()

@@ -571,7 +571,7 @@ static void *matvec_job(void *p) {
 }
 
 /* nthreads 0: the cores this process may run on (rayon's default pool),
- * capped by GQO_MAX_THREADS (default 16, the GPU box's CPU share). */
+ * capped by GQO_MAX_THREADS (default 16, one GPU's share of a host). */
 static int hw_threads(int n) {
     if (n > 0) return n;
     cpu_set_t set;

@@ -144,7 +144,7 @@ def qwen7b(backend):
 
 @pytest.mark.timeout(600)
 def test_generate_qwen25_7b_constant_stream(qwen7b):
-    """BASELINE configs[3] with its specified distributions: 4096 cached
+    """The 28-layer 7B decode with its specified distributions: 4096 cached
     positions, greedy steps.  The Q4_K blocks' positive mean (d*sc*7.5 -
     dmin*m per element) gives every gate/up row a bias along the input's sum
     and the residual's common component grows to ~1e11 over the layers, so
@@ -251,7 +251,7 @@ def test_qwen25_7b_live_stream_depends_on_every_layer(qwen7b_live):
 
 @pytest.mark.timeout(600)
 def test_generate_qwen25_7b_live_uploaded(qwen7b_live):
-    """BASELINE configs[3]: 4096 uploaded f16 rows (KvCache::write_range),
+    """4096 uploaded f16 rows (KvCache::write_range),
     then 128 greedy steps.  The first step's logits agree to LOGIT_TOL, all
     128 tokens equal the oracle's (cpu_path.rs:695-818, sampler.rs:120-131),
     and the 128 K/V rows every one of the 28 layers wrote agree with the

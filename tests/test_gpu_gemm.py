@@ -345,7 +345,7 @@ def test_gemm_bf16_q8_0_q5k(backend, orc, dtype, rows, k, n):
     """WeightMap::matmul_batch_into (src/model/mod.rs:414-464) dequantizes
     every dtype with dequant_row; the bf16 GEMM of Q8_0 and Q5_K weights
     against the same-operand fp64 product (1e-4) and the fp32 CPU path
-    (1e-2, bf16 operands).  (8192 x 2048 is BASELINE configs[0]'s Q8_0 FFN-up
+    (1e-2, bf16 operands).  (8192 x 2048 is the 1B-class Q8_0 FFN-up
     matrix, here over 512 prompt tokens.)"""
     import gq
     say(f"gemm bf16 dtype={dtype} rows={rows} k={k} n={n}")

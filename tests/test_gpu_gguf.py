@@ -132,7 +132,7 @@ def test_gguf_upload_tensor_matvec(backend, tmp_path, dtype):
 
 
 def test_gguf_q8_0_model_prefill_and_generate(backend, tmp_path):
-    """An all-Q8_0 file (the file type of BASELINE configs[0]'s Llama-3.2-1B
+    """An all-Q8_0 file (the file type of the Llama-3.2-1B
     Q8_0 model; here a small decoder with a Q8_0 head): gq_model_prefill of
     a 40-token prompt (LlamaModel::run_batch, cpu_path.rs:834-991) against
     the oracle stepping the same tokens (logits to the bf16-operand bound

@@ -71,7 +71,7 @@ def _f16(a):
 
 
 # Projection-type mixes beyond Q4_K_M: an all-Q8_0 model (the Llama-3.2-1B
-# Q8_0 file type of BASELINE configs[0]) and a Q5_K_M-like one.
+# Q8_0 file type of 1B-class files) and a Q5_K_M-like one.
 MIXES = {"Q4_K_M": {}, "Q8_0": dict(attn_type=syn.Q8_0, gate_up_type=syn.Q8_0, down_type=syn.Q8_0,
                                     head_type=syn.Q8_0),
          "Q5_K_M": dict(attn_type=syn.Q5_K, gate_up_type=syn.Q5_K, down_type=syn.Q6_K)}
