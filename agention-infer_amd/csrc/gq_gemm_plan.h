@@ -58,37 +58,54 @@ inline int gemm_quad_nt(int n) {
 // in all) with K in ks parts: rounds of blocks (one a CU), each a start, its
 // quads' dequant and MFMAs, and what of their weights' way from HBM these do not
 // cover (longer the more of the CUs load at once); a split adds the reduction's
-// launch and writes and reads ks partial products.  The constants are those
-// that choose best, here and in gemm_quad_faster, over 9860 measured calls of 1
-// to 128 tokens on 64 x 256 to 128256 x 2048 weights; of the times themselves
-// they miss 11% on average.
+// launch and writes and reads ks partial products.  The constants (the types
+// differ in the dequant and in what a block's first loads wait for) are those that
+// choose best, here and in gemm_quad_faster, over every split of 4100 calls of 1 to
+// 128 tokens on 64 x 256 to 130000 x 256 weights: the chosen ones take 0.1% longer
+// than the best on average, 22 of them more than 5%, the worst 12%.  Of the times
+// themselves they miss 11%.
 inline double gemm_quad_time(int dtype, int tiles, long rows, int units, int n, int ks, int num_cus) {
   const int nt = gemm_quad_nt(n), quads = ((units + 3) / 4 + ks - 1) / ks;
   const double rounds = (double)(((long)tiles * ks + num_cus - 1) / num_cus), fill = tiles * ks / (rounds * num_cus);
   const double bits = dtype == 12 ? 4.5 : dtype == 13 ? 5.5 : dtype == 14 ? 6.5625 : 8.5;
   const double hbm = fill * num_cus * GEMM_QUAD_ROWS * 256 * bits / 8 / 4.7e6;  // a unit of every block
-  const double step = (dtype == 12 ? 2.85 : dtype == 8 ? 2.7 : 3.4) + 0.75 * nt;
+  const double start = dtype == 12 ? 0.76 : dtype == 14 ? 1.34 : 0.91;
+  const double step = (dtype == 13 ? 2.56 : dtype == 8 ? 2.81 : 2.7) + 0.683 * nt;
   const double out = (double)rows * n * 8e-6 / 4.5;  // a result written and read
-  return 4.7 + rounds * (0.9 + 0.11 * hbm * std::min(4 * quads, units) + step * quads) +
-         (ks > 1 ? 2.85 + 1.1 * ks * out : 0.0) + 0.58 * out;
+  return 4.76 + rounds * (start + 0.135 * hbm * std::min(4 * quads, units) + step * quads) +
+         (ks > 1 ? 2.23 + 0.053 * ks + 1.03 * ks * out : 0.0) + 0.463 * out;
 }
 
-// The K split (over quads) of such a call: the least estimated time.  Measured
-// unsplit / in 2, us a call: 3584 x 2048 Q8_0 at 128 tokens 22.6 / 19.1, 9000 x
-// 2048 Q4_K at 128 23.5 / 24.2, 14336 x 2048 Q4_K at 128 24.8 / 28.5, 65536 x
-// 3584 Q6_K at 64 93.4 / 103.8 (the partial products' traffic); 3584 x 18944
-// Q6_K at 37 107 unsplit, 50 in 3, 36 in 5, 32 in 8, 41 in 10 (a second round).
+// The K split (over quads) of such a call: the least estimated time.  Up to 32
+// tokens (two token tiles) many splits lie closer together than the estimates'
+// error, and the split with the least rounds of quads, a start and a reduction
+// counted as parts of one, is right more often: there that one, unless another's
+// time is 3% less.  (Of 5700 calls 13 took 3% to 13% longer by the estimates alone
+// than by the count; now three do, by up to 5%.)  Measured unsplit / in 2, us a
+// call: 3584 x 2048 Q8_0 at 128 tokens 22.0 / 18.4, 14336 x 2048 Q4_K at 128 22.8 /
+// 26.4, 65536 x 3584 Q6_K at 128 128.6 / 136.7 (the partial products' traffic);
+// 3584 x 18944 Q6_K at 37 107 unsplit, 50 in 3, 36 in 5, 32 in 8, 41 in 10 (a second
+// round); 12071 x 6912 Q6_K at 24 40.1 unsplit, 30.5 in 2, 36.3 in 7 (three rounds
+// of single quads).
 inline int gemm_quad_ksplit(int dtype, int tiles, long rows, int units, int n, int num_cus) {
-  int best = 1;
-  double best_t = 1e30;
-  for (int ks = 1; ks <= std::min((units + 3) / 4, 16); ks++) {
+  const int quads = (units + 3) / 4;
+  int best = 1, count = 1;
+  double best_t = 1e30, count_t = 1e30, time_of_count = 0.0;
+  for (int ks = 1; ks <= std::min(quads, 16); ks++) {
     const double t = gemm_quad_time(dtype, tiles, rows, units, n, ks, num_cus);
+    const long rounds = ((long)tiles * ks + num_cus - 1) / num_cus;
+    const double c = rounds * (0.5 + (quads + ks - 1) / ks) + (ks > 1 ? 0.7 + 0.05 * ks : 0.0);
     if (t < best_t - 1e-9) {
       best_t = t;
       best = ks;
     }
+    if (c < count_t - 1e-9) {
+      count_t = c;
+      count = ks;
+      time_of_count = t;
+    }
   }
-  return best;
+  return n > 32 || best_t < 0.97 * time_of_count ? best : count;
 }
 
 // The 160 x 256 kernel's K split of a launch with this many row x token tiles and
@@ -126,9 +143,9 @@ inline double gemm_direct_time(int dtype, int rows, int units, int n, int num_cu
 // up to four times, but where a row is one unit, and three quarters of the MFMA
 // depth its zeros, or where its lower tiles take one round of blocks more; then
 // the estimates decide.  Measured short / 160 x 256, us a call: 4800 x 256 Q4_K
-// at 64 tokens 12.3 / 12.5, at 97 15.7 / 12.7; 37888 x 256 Q8_0 (339 and 237
-// tiles) at 1 token 14.4 / 12.0, at 128 27.7 / 15.1; 37888 x 512 Q6_K at 32 18.8 /
-// 18.8, at 128 32.1 / 21.5; 18944 x 512 Q4_K at 128 17.9 / 26.2.
+// at 64 tokens 10.8 / 12.0, at 97 13.8 / 12.1; 37888 x 256 Q8_0 (339 and 237
+// tiles) at 1 token 13.9 / 10.9, at 128 27.3 / 15.0; 37888 x 512 Q6_K at 128 28.1 /
+// 21.3; 18944 x 512 Q4_K at 128 15.5 / 25.9.
 inline bool gemm_quad_faster(int dtype, int rows, int units, int n, int num_cus) {
   const int tiles = (rows + GEMM_QUAD_ROWS - 1) / GEMM_QUAD_ROWS;
   const int rounds = (tiles + num_cus - 1) / num_cus, direct = ((rows + 159) / 160 + num_cus - 1) / num_cus;

@@ -5,7 +5,7 @@ Q8_0, Q4_K, Q5_K, Q6_K = 8, 12, 13, 14
 # Batches of up to 128 tokens on the 160 x 256 bf16 kernel: one unit a row, one
 # and several row tiles with and without a ragged last one, ragged units.
 BF16_SHORT_DIRECT = [
-    (Q4_K, 480, 256, 97), (Q5_K, 4785, 256, 128), (Q6_K, 14335, 256, 113), (Q8_0, 4800, 224, 128),
+    (Q4_K, 480, 256, 97), (Q5_K, 30001, 250, 128), (Q6_K, 14335, 256, 113), (Q8_0, 4800, 224, 128),
     (Q4_K, 37888, 131, 33), (Q8_0, 37889, 512, 128),
 ]
 

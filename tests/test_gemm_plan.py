@@ -34,12 +34,12 @@ def units(k):
 # bf16 calls: (dtype, rows, k, tokens, us on the short-batch kernel, us on the
 # 160 x 256 one).
 SHORT_TIMES = [
-    (Q4_K, 4800, 256, 64, 12.3, 12.5), (Q4_K, 4800, 256, 97, 15.7, 12.7), (Q4_K, 9000, 256, 64, 12.4, 14.9),
-    (Q6_K, 18944, 256, 128, 18.1, 15.6), (Q8_0, 9000, 256, 64, 11.5, 14.7), (Q5_K, 14336, 256, 128, 17.7, 15.5),
-    (Q6_K, 1200, 256, 16, 11.6, 12.9), (Q6_K, 4800, 512, 128, 16.8, 18.6), (Q4_K, 18944, 512, 128, 17.9, 26.2),
-    (Q4_K, 18944, 3584, 64, 29.8, 45.9), (Q4_K, 37888, 256, 32, 14.4, 12.7), (Q8_0, 37888, 256, 1, 14.4, 12.0),
-    (Q8_0, 37888, 256, 128, 27.7, 15.1), (Q6_K, 37888, 512, 128, 32.1, 21.5), (Q4_K, 37888, 1024, 128, 32.1, 28.7),
-    (Q6_K, 65536, 256, 64, 31.1, 25.1), (Q8_0, 65536, 512, 112, 41.6, 33.7), (Q8_0, 128256, 256, 96, 54.4, 42.9),
+    (Q4_K, 4800, 256, 64, 10.8, 12.0), (Q4_K, 4800, 256, 97, 13.8, 12.1), (Q4_K, 9000, 256, 64, 10.6, 14.0),
+    (Q6_K, 18944, 256, 128, 15.9, 15.1), (Q8_0, 9000, 256, 64, 10.6, 13.8), (Q5_K, 14336, 256, 128, 15.3, 15.0),
+    (Q6_K, 1200, 256, 16, 9.0, 11.8), (Q6_K, 4800, 512, 128, 14.7, 18.4), (Q4_K, 18944, 512, 128, 15.5, 25.9),
+    (Q4_K, 18944, 3584, 64, 28.2, 44.6), (Q4_K, 37888, 256, 32, 13.2, 12.1), (Q8_0, 37888, 256, 1, 13.8, 10.9),
+    (Q8_0, 37888, 256, 128, 27.3, 15.0), (Q6_K, 37888, 512, 128, 28.1, 21.3), (Q4_K, 37888, 1024, 128, 28.4, 28.3),
+    (Q6_K, 65536, 256, 64, 28.2, 24.3), (Q8_0, 65536, 512, 112, 40.1, 33.1), (Q8_0, 128256, 256, 96, 53.4, 42.0),
 ]
 
 
@@ -69,12 +69,27 @@ Q6_TIMES = [
 # bf16 calls on the short-batch kernel: (dtype, rows, k, tokens, us unsplit, us in
 # 2 K splits).
 SPLIT_TIMES = [
-    (Q4_K, 3584, 1280, 128, 23.9, 20.5), (Q4_K, 4800, 1280, 96, 20.6, 18.7), (Q8_0, 3584, 2048, 128, 22.6, 19.0),
-    (Q8_0, 4800, 2048, 96, 19.9, 17.6), (Q8_0, 9000, 2048, 48, 16.6, 15.5), (Q4_K, 14336, 2048, 48, 16.4, 17.3),
-    (Q8_0, 14336, 2048, 96, 22.3, 24.1), (Q8_0, 14336, 2048, 128, 25.8, 28.1), (Q8_0, 14336, 1280, 128, 23.9, 26.4),
-    (Q6_K, 37888, 3584, 48, 55.9, 58.7), (Q4_K, 37888, 3584, 96, 69.2, 72.4), (Q8_0, 65536, 3584, 64, 99.5, 107.8),
-    (Q4_K, 14336, 2048, 96, 21.0, 24.0), (Q4_K, 14336, 2048, 128, 24.8, 28.5), (Q6_K, 65536, 3584, 128, 132.6, 147.2),
-    (Q8_0, 65536, 3584, 128, 138.0, 149.4), (Q6_K, 37888, 4096, 64, 63.7, 68.2), (Q4_K, 37888, 4096, 128, 82.6, 86.1),
+    (Q4_K, 3584, 1280, 128, 21.6, 18.2), (Q4_K, 4800, 1280, 96, 18.9, 16.9), (Q8_0, 3584, 2048, 128, 22.0, 18.4),
+    (Q8_0, 4800, 2048, 96, 19.4, 16.9), (Q8_0, 9000, 2048, 48, 15.2, 14.9), (Q4_K, 14336, 2048, 48, 14.8, 15.9),
+    (Q8_0, 14336, 2048, 96, 22.2, 23.6), (Q8_0, 14336, 2048, 128, 25.4, 27.6), (Q8_0, 14336, 1280, 128, 23.6, 25.9),
+    (Q6_K, 37888, 3584, 48, 53.6, 55.5), (Q4_K, 37888, 3584, 96, 66.0, 67.6), (Q8_0, 65536, 3584, 64, 97.8, 103.7),
+    (Q4_K, 14336, 2048, 96, 19.3, 22.4), (Q4_K, 14336, 2048, 128, 22.8, 26.4), (Q6_K, 65536, 3584, 128, 128.6, 136.7),
+    (Q8_0, 65536, 3584, 128, 134.1, 142.9), (Q6_K, 37888, 4096, 64, 60.9, 64.2), (Q4_K, 37888, 4096, 128, 79.2, 81.4),
+]
+
+
+# (dtype, rows, k, tokens, us in 1, 2, ... splits): few tokens, where rounds of
+# single quads are slower than their count tells.
+SPLITS_TIMES = [
+    (Q6_K, 9886, 8192, 3, [42.2, 27.8, 38.8, 30.9, 31.0, 41.9, 42.3, 31.5]),
+    (Q8_0, 171, 12192, 25, [57.5, 34.0, 25.5, 21.9, 22.1, 18.5, 19.1, 19.4, 20.3, 20.4, 20.4, 17.4]),
+    (Q6_K, 12071, 6912, 24, [40.1, 30.5, 41.5, 34.1, 43.7, 45.4, 36.3]),
+    (Q6_K, 14976, 7680, 10, [42.2, 47.9, 39.4, 42.5, 42.2, 52.7, 51.7, 45.0]),
+    (Q5_K, 12198, 6400, 21, [41.4, 30.9, 41.9, 34.1, 44.0, 44.9, 35.1]),
+    (Q6_K, 14618, 7680, 3, [41.8, 48.0, 40.0, 43.0, 42.7, 52.3, 52.4, 45.4]),
+    (Q6_K, 10396, 13056, 2, [64.1, 42.0, 56.2, 48.0, 40.9, 54.7, 43.7, 43.7, 48.2, 48.8, 49.1, 55.2, 46.4]),
+    (Q8_0, 12266, 1152, 24, [15.4, 14.0]),
+    (Q4_K, 14105, 2304, 9, [17.4, 16.0, 16.0]),
 ]
 
 
@@ -84,6 +99,9 @@ def test_quad_split_rule(ask):
     got = ask([f"quad {t} {r} {units(k)} {n}" for t, r, k, n, _, _ in SPLIT_TIMES])
     for (t, r, k, n, one, two), (ks,) in zip(SPLIT_TIMES, ((g[0],) for g in got)):
         assert {1: one, 2: two}[ks] <= 1.1 * min(one, two), f"dtype {t}, {r} x {k} at {n} tokens: {ks} splits"
+    got = ask([f"quad {t} {r} {units(k)} {n}" for t, r, k, n, _ in SPLITS_TIMES])
+    for (t, r, k, n, us), g in zip(SPLITS_TIMES, got):
+        assert us[g[0] - 1] <= 1.05 * min(us), f"dtype {t}, {r} x {k} at {n} tokens: {g[0]} splits"
 
 
 def test_q6_small_rule(ask):
