@@ -166,8 +166,8 @@ struct Q8Plan {
 // The K split with the least estimated time of a token tile, us: rounds of
 // blocks, each a start and its units (6.5 or 10 us each), and the reduction's
 // launch and traffic.  Measured with 128- / 256-token tiles, us a call: 18944
-// x 3584 Q4_K at 512 tokens 197 / 142, at 128 62 / 74; 3584 x 18944 Q6_K at
-// 200 139 / 99; 9000 x 512 Q6_K at 300 26 / 31; 3584 x 3584 Q4_K at 512 61 / 48
+// x 3584 Q4_K at 512 tokens 177 / 124, at 128 57 / 72; 3584 x 18944 Q6_K at
+// 200 135 / 94; 9000 x 512 Q6_K at 300 23 / 30; 3584 x 3584 Q4_K at 512 58 / 47
 // (in 2 / 5 splits).
 inline double q8_split(int rows, int units, int nj, int n, int num_cus, int &ksplit) {
   const double out = (double)n * rows * 8e-6 / 4.5;  // one partial product written and read
@@ -191,8 +191,8 @@ inline double q8_split(int rows, int units, int nj, int n, int num_cus, int &ksp
 // blocks wait on latency, 4 us a unit, until they are more than the CUs; the
 // other kernel pays a longer start, its 160-row stages and (in p's split) a
 // reduction.  Measured small / 160-row, at 256 CUs: 600 x 256 at 200 tokens 11 /
-// 19, 4800 x 512 at 200 18 / 26, 2400 x 768 at 700 26 / 35, 9000 x 256 at 512
-// 26 / 22, 1200 x 1024 at 1024 31 / 28, 600 x 1024 at 8 22 / 17.
+// 16, 4800 x 512 at 200 17 / 23, 2400 x 768 at 700 25 / 33, 9000 x 256 at 512
+// 27 / 19, 9000 x 512 at 700 44 / 32, 600 x 1024 at 16 21 / 16.
 inline bool q6_small(int rows, int units, int n, const Q8Plan &p, int num_cus) {
   const double out = (double)n * rows * 8e-6 / 4.5;
   const long blocks = (long)((rows + Q6S - 1) / Q6S) * ((n + Q6S - 1) / Q6S);

@@ -418,7 +418,7 @@ __global__ __launch_bounds__(512) void k_gemm_q8(Q8Args a) {
 // unit (PROD: y += (d xs) D).  A stage ahead of its use, threads 0-127 turn
 // the quants of (row tid / 2, half tid % 2) into A fragments, 128-191 write the
 // row's scales and d, and all of them the stage's X fragments and scales.
-// 600 x 256 x 200: 11 us a call, 19 on the kernel above; 4800 x 512 x 200: 18 and 26.
+// 600 x 256 x 200: 11 us a call, 16 on the kernel above; 4800 x 512 x 200: 17 and 23.
 template <bool PROD>
 __global__ __launch_bounds__(256) void k_gemm_q6_small(Q8Args a) {
   constexpr int NJ = Q6S / 16;

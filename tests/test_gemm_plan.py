@@ -54,15 +54,15 @@ def test_quad_kernel_rule(ask):
 # Q6_K int8 calls: (rows, k, tokens, us on the 64 x 64 blocks, us on the
 # 160-row ones with their K split).
 Q6_TIMES = [
-    (64, 256, 2, 11.2, 15.9), (133, 256, 200, 11.1, 19.7), (600, 256, 200, 11.3, 19.2),
-    (2400, 256, 128, 11.4, 20.3), (4800, 256, 300, 13.9, 21.1), (9000, 256, 512, 26.1, 21.5),
-    (14336, 256, 64, 11.4, 18.1), (18944, 256, 384, 33.3, 25.8), (133, 512, 2, 12.7, 16.5),
-    (1200, 512, 512, 15.5, 22.8), (4800, 512, 200, 17.5, 26.1), (9000, 512, 384, 29.2, 26.7),
-    (9000, 512, 700, 43.6, 31.9), (2400, 768, 700, 25.6, 35.6), (4800, 768, 300, 25.0, 34.3),
-    (9000, 768, 700, 58.2, 42.7), (14336, 768, 200, 34.6, 34.9), (64, 1024, 2, 20.6, 16.2),
-    (600, 1024, 16, 21.5, 17.1), (2400, 1024, 300, 23.8, 27.4), (4800, 1024, 300, 30.4, 35.1),
-    (9000, 1024, 512, 55.6, 44.2), (9000, 1280, 300, 44.2, 50.0), (133, 2048, 64, 38.1, 19.5),
-    (3584, 2048, 512, 52.7, 50.4), (3584, 3072, 64, 55.7, 30.0),
+    (64, 256, 2, 8.2, 15.1), (133, 256, 200, 9.9, 16.0), (600, 256, 200, 11.0, 16.4), (2400, 256, 128, 10.9, 17.6),
+    (4800, 256, 300, 13.8, 18.2), (9000, 256, 512, 26.6, 19.3), (14336, 256, 64, 10.9, 16.5),
+    (18944, 256, 384, 33.8, 25.6), (133, 512, 2, 12.1, 14.7), (1200, 512, 512, 15.4, 20.0),
+    (4800, 512, 200, 17.1, 23.3), (9000, 512, 384, 29.9, 24.1), (9000, 512, 700, 43.7, 31.8),
+    (2400, 768, 700, 24.8, 32.6), (4800, 768, 300, 24.5, 31.4), (9000, 768, 700, 57.6, 42.5),
+    (14336, 768, 200, 34.0, 31.9), (64, 1024, 2, 20.2, 15.8), (600, 1024, 16, 21.3, 16.4),
+    (2400, 1024, 300, 23.7, 24.7), (4800, 1024, 300, 30.1, 32.5), (9000, 1024, 512, 54.9, 40.4),
+    (9000, 1280, 300, 43.5, 46.7), (133, 2048, 64, 37.3, 17.3), (3584, 2048, 512, 53.6, 47.8),
+    (3584, 3072, 64, 54.6, 28.3),
 ]
 
 
