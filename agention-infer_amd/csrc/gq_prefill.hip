@@ -586,6 +586,21 @@ __global__ __launch_bounds__(512) void k_attn_prefill(const float *q, const uint
 // ------------------------------------------------------------------ host
 static int round_up(int v, int m) { return (v + m - 1) / m * m; }
 
+// The launch of q, k, v that begins with matrix i: itself and the later ones of its
+// type (with their outputs, unless null), marked in `done`; their count, 0 if i is done.
+static int same_type(const gq_weight *const *qkv, int i, int &done, const gq_weight **grp, float *const *outs,
+                     float **gout) {
+  if (done >> i & 1) return 0;
+  int c = 0;
+  for (int j = i; j < 3; j++) {
+    if (done >> j & 1 || qkv[j]->L.dtype != qkv[i]->L.dtype) continue;
+    if (outs) gout[c] = outs[j];
+    grp[c++] = qkv[j];
+    done |= 1 << j;
+  }
+  return c;
+}
+
 // The largest partial buffer of any launch of a pass of up to nmax tokens (the K
 // split depends on the batch, past GEMM_QUAD_MAX tokens on its token tiles).
 size_t prefill_part_floats(const DecodeLaunch &m, int nmax, int num_cus) {
@@ -603,14 +618,10 @@ size_t prefill_part_floats(const DecodeLaunch &m, int nmax, int num_cus) {
   for (int n = 1;; n = std::min(n < GEMM_QUAD_MAX ? n + 1 : n + 16, nmax)) {
     const bool quad = n <= GEMM_QUAD_MAX;
     for (int L : layers) {
-      const gq_weight *qkv[3] = {m.wq[L], m.wk[L], m.wv[L]};
-      for (int set = 1; set < 8; set++) {  // whichever of them share a type and so a launch
-        const gq_weight *grp[3];
-        int c = 0;
-        for (int i = 0; i < 3; i++)
-          if (set >> i & 1) grp[c++] = qkv[i];
-        best = std::max(best, gemm_part_floats(grp, c, n, quad, num_cus, false));
-      }
+      const gq_weight *qkv[3] = {m.wq[L], m.wk[L], m.wv[L]}, *grp[3];
+      for (int i = 0, done = 0; i < 3; i++)
+        if (const int c = same_type(qkv, i, done, grp, nullptr, nullptr))
+          best = std::max(best, gemm_part_floats(grp, c, n, quad, num_cus, false));
       best = std::max(best, gemm_part_floats(&m.wo[L], 1, n, quad, num_cus, true));
       const gq_weight *gu[2] = {m.wgate[L], m.wup[L]};
       best = std::max(best, gemm_part_floats(gu, 2, n, quad, num_cus, false));
@@ -637,20 +648,11 @@ hipError_t launch_prefill(const DecodeLaunch &m, const PrefillBufs &b, const int
                        round_up(H, kq), quad, m.eps, b.xb, b.part, pending);
     pending = 0;
     // q, k, v: one launch per distinct dtype (attn_v is Q6_K in some files)
-    const gq_weight *qkv[3] = {m.wq[L], m.wk[L], m.wv[L]};
-    float *outs[3] = {b.q, b.k, b.v};
-    bool done[3] = {false, false, false};
-    for (int i = 0; i < 3; i++) {
-      if (done[i]) continue;
-      const gq_weight *grp[3];
-      float *gout[3];
-      int c = 0;
-      for (int j = i; j < 3; j++)
-        if (!done[j] && qkv[j]->L.dtype == qkv[i]->L.dtype) {
-          grp[c] = qkv[j];
-          gout[c++] = outs[j];
-          done[j] = true;
-        }
+    const gq_weight *qkv[3] = {m.wq[L], m.wk[L], m.wv[L]}, *grp[3];
+    float *outs[3] = {b.q, b.k, b.v}, *gout[3];
+    for (int i = 0, done = 0; i < 3; i++) {
+      const int c = same_type(qkv, i, done, grp, outs, gout);
+      if (!c) continue;
       if ((e = launch_gemm_bf16(grp, gout, c, b.xb, n, quad, b.part, false, num_cus, s)) != hipSuccess) return e;
     }
     uint16_t *kc, *vc;  // the f16 K/V rows the attention reads
