@@ -285,7 +285,7 @@ def test_gemm_odd_rows(backend, mode, dtype, rows, k, n):
         buf = torch.full((n * r + 9,), 7.0, device="cuda")
         Y = buf[1:1 + n * r].view(n, r)
         t = []
-        for i in range(6):
+        for _ in range(12):
             a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
             a.record()
             for _ in range(20):
